@@ -356,6 +356,30 @@ int ulm_decode_read(const float *S, const float *pv, const float *cj, int m, con
 int ulm_decode_flush(float *S, const float *pv, const float *pr, int m, const float *q, const float *g,
                      const float *x, const float *ymu, float *out, int N, int D, int A, void *stream);
 
+/* One position of n_layers consecutive blocks for up to 256 sequences whose
+ * states are small (up to 320 MB per block), two launches per block (a third
+ * where a block's 16th term makes it write its state back): what the per-kernel entries above and the three projections
+ * compute, on the same deferred state. x (N,D) is the first block's input,
+ * out (N,D) the last one's output, neither aliasing the other.
+ * A layer names a block's parameters, fp32 and contiguous: norm_w (D,),
+ * conv_w (D,Kc), key_w (A,D), key_b (A,), log_eps (1,), val_w (D,D),
+ * mu_w (D,A), the prior mass w (A,) and g = log lam (1,); and its state:
+ * conv_buf (N,D,Kc-1), S (N,D,A) = S_base, c (N,A) and r_prev (N,A), updated in
+ * place, and the pending values pv (16,N,D) and keys pr (16,N,A), of which
+ * `pending` (0 .. 15) are held. The position appends one; a block that held 15
+ * is written back and holds none afterwards. mu_w, w, S, c and r_prev 16-byte
+ * aligned; A % 4 == 0, A <= 4096, Kc <= 8. Workspace of
+ * ulm_decode_step_workspace_bytes() bytes (0: sizes this form does not take). */
+typedef struct ulm_decode_layer {
+    const float *norm_w, *conv_w, *key_w, *key_b, *log_eps, *val_w, *mu_w, *w, *g;
+    float *conv_buf, *S, *c, *r_prev, *pv, *pr;
+    double norm_eps;
+    long long pending;
+} ulm_decode_layer;
+size_t ulm_decode_step_workspace_bytes(int N, int D, int A, int Kc);
+int ulm_decode_step(const ulm_decode_layer *layers, int n_layers, const float *x, float *out, void *workspace,
+                    size_t workspace_bytes, int N, int D, int A, int Kc, void *stream);
+
 /* ------------------------------------------------------------------------
  * Diagnostics: HIP-event timing of every chunked-kernel launch (ulm_la and
  * the launches inside ulm_fm_fwd / ulm_fm_bwd) between start and stop, on

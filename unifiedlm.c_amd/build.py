@@ -20,7 +20,7 @@ LIB = os.path.join(HERE, "libulm_fm.so")
 PROBE_LIB = os.path.join(HERE, "libulm_probe.so")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 
-SOURCES = ["status.hip", "elementwise.hip", "decode.hip", "address.hip", "fm_stats.hip", "fm_chunk.hip", "pair.hip",
+SOURCES = ["status.hip", "elementwise.hip", "decode.hip", "decode_step.hip", "address.hip", "fm_stats.hip", "fm_chunk.hip", "pair.hip",
            "fm_chunks.hip", "la_kgroup.hip", "fm_ops.hip", "block.hip", "wgrad.hip"]
 PROBE_SOURCES = ["status.hip", "probe.hip"]   # the test-only probe library
 ARCH = "gfx950"

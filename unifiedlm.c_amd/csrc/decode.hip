@@ -346,7 +346,12 @@ __global__ __launch_bounds__(256) void decode_read_kernel(const float *__restric
     }
 }
 
-constexpr int kFlushRows = 64;   // rows (features) per workgroup
+// Rows (features) per workgroup of a write-back: 64 where that leaves 1024
+// workgroups (each re-reads its sequence's pending keys, 12 KB a key at 3072
+// slots), else 8, since fewer workgroups leave CUs idle: at 8 sequences of the
+// 110M widths 64 rows make 96 workgroups and the launch took 76 us for 150 MB.
+constexpr int kFlushRows = 64, kFlushRowsFew = 8;
+constexpr int kFlushWgs = 1024;
 // rows whose loads a lane has in flight at once: 8 where the registers allow
 // (12 waves, 168 VGPRs), else 4
 template <int MAXW> constexpr int flush_batch() { return MAXW <= 12 ? 8 : 4; }
@@ -354,27 +359,28 @@ template <int MAXW> constexpr int flush_batch() { return MAXW <= 12 ? 8 : 4; }
 // Flush position: S_base[n, d, :] <- lam^m S_base + sum_j lam^(m-1-j) pv_j[n, d] rp_j[n, :],
 // out[n, d] = x + S_base . q + ymu. Column-strip layout: wave w of the
 // workgroup owns slots 256 w .. 256 w + 255 (one 16-byte slice per lane) of
-// kFlushRows rows of one sequence, and keeps its slices of the m pending keys
+// ROWS rows of one sequence, and keeps its slices of the m pending keys
 // and of q in registers for all of them; the per-row coefficients
 // lam^(m-1-j) pv_j[n, d] are uniform over the wave. Each lane streams its
 // slice of a batch of rows at a time (loads first), and the rows' dot
 // products are summed over the waves through LDS in a fixed order.
+// Without OUT only the state is written (q, x, ymu and out are not read).
 // A <= 64 MAXW (MAXW waves at most), A % 4 == 0; MAXW = 12 (A <= 3072) allows
 // 168 VGPRs per lane, where the 16 key slices fit without spills.
-template <int MAXW>
+template <int MAXW, int ROWS, bool OUT>
 __global__ __launch_bounds__(MAXW * 64) void decode_flush_kernel(float *__restrict__ S, const float *__restrict__ pv,
                                                             const float *__restrict__ pr, int m,
                                                             const float *__restrict__ q, const float *__restrict__ g,
                                                             const float *__restrict__ x, const float *__restrict__ ymu,
                                                             float *__restrict__ out, int N, int D, int A) {
-    __shared__ float part[16][kFlushRows];
-    __shared__ float spv[kMaxPending][kFlushRows];   // the block's rows' pending values
+    __shared__ float part[16][ROWS];
+    __shared__ float spv[kMaxPending][ROWS];   // the block's rows' pending values
     const size_t n = blockIdx.x;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave, nw = blockDim.x / kWave;
-    const int d0 = blockIdx.y * kFlushRows;
-    for (int k = threadIdx.x; k < kMaxPending * kFlushRows; k += blockDim.x) {
-        const int j = k / kFlushRows, d = min(d0 + k % kFlushRows, D - 1);
-        spv[j][k % kFlushRows] = j < m ? pv[(static_cast<size_t>(j) * N + n) * D + d] : 0.f;
+    const int d0 = blockIdx.y * ROWS;
+    for (int k = threadIdx.x; k < kMaxPending * ROWS; k += blockDim.x) {
+        const int j = k / ROWS, d = min(d0 + k % ROWS, D - 1);
+        spv[j][k % ROWS] = j < m ? pv[(static_cast<size_t>(j) * N + n) * D + d] : 0.f;
     }
     const int A4 = A / 4, i = wave * kWave + lane;   // this lane's 16-byte slice of every row
     const bool ok = i < A4;
@@ -383,12 +389,12 @@ __global__ __launch_bounds__(MAXW * 64) void decode_flush_kernel(float *__restri
 #pragma unroll
     for (int j = 0; j < kMaxPending; ++j)
         rp[j] = reinterpret_cast<const f32x4 *>(pr + (static_cast<size_t>(j < m ? j : 0) * N + n) * A)[ic];
-    const f32x4 qv = reinterpret_cast<const f32x4 *>(q + n * A)[ic];
+    const f32x4 qv = OUT ? reinterpret_cast<const f32x4 *>(q + n * A)[ic] : f32x4{0.f, 0.f, 0.f, 0.f};
     const float lam = __expf(g[0]);
     float lm = 1.f;
     for (int j = 0; j < m; ++j) lm *= lam;
     __syncthreads();
-    for (int b = 0; b < kFlushRows; b += flush_batch<MAXW>()) {
+    for (int b = 0; b < ROWS; b += flush_batch<MAXW>()) {
         f32x4 sv[flush_batch<MAXW>()];
 #pragma unroll
         for (int u = 0; u < flush_batch<MAXW>(); ++u) {
@@ -411,14 +417,17 @@ __global__ __launch_bounds__(MAXW * 64) void decode_flush_kernel(float *__restri
             for (int j = 0; j < kMaxPending; ++j) t += cf[j] * rp[j];
             if (ok && d < D)
                 __builtin_nontemporal_store(t, reinterpret_cast<f32x4 *>(S + (n * D + d) * static_cast<size_t>(A)) + i);
-            const f32x4 pq = t * qv;
-            float acc = ok ? (pq[0] + pq[1]) + (pq[2] + pq[3]) : 0.f;
-            acc = wave_sum(acc);
-            if (lane == 0) part[wave][b + u] = acc;
+            if constexpr (OUT) {
+                const f32x4 pq = t * qv;
+                float acc = ok ? (pq[0] + pq[1]) + (pq[2] + pq[3]) : 0.f;
+                acc = wave_sum(acc);
+                if (lane == 0) part[wave][b + u] = acc;
+            }
         }
     }
+    if constexpr (!OUT) return;
     __syncthreads();
-    if (threadIdx.x < kFlushRows) {
+    if (threadIdx.x < ROWS) {
         const int d = d0 + threadIdx.x;
         if (d < D) {
             float y = 0.f;
@@ -426,6 +435,33 @@ __global__ __launch_bounds__(MAXW * 64) void decode_flush_kernel(float *__restri
             out[n * D + d] = x[n * D + d] + y + ymu[n * D + d];
         }
     }
+}
+
+namespace {
+template <bool OUT>
+int launch_flush(float *S, const float *pv, const float *pr, int m, const float *q, const float *g, const float *x,
+                 const float *ymu, float *out, int N, int D, int A, hipStream_t s) {
+    const int waves = (A / 4 + kWave - 1) / kWave;   // one 256-slot strip per wave
+    const bool few = static_cast<size_t>(N) * ((D + kFlushRows - 1) / kFlushRows) < kFlushWgs;
+    const int rows = few ? kFlushRowsFew : kFlushRows;
+    const dim3 grid(N, (D + rows - 1) / rows), wg(waves * kWave);
+    if (waves <= 12 && few)
+        decode_flush_kernel<12, kFlushRowsFew, OUT><<<grid, wg, 0, s>>>(S, pv, pr, m, q, g, x, ymu, out, N, D, A);
+    else if (waves <= 12)
+        decode_flush_kernel<12, kFlushRows, OUT><<<grid, wg, 0, s>>>(S, pv, pr, m, q, g, x, ymu, out, N, D, A);
+    else if (few)
+        decode_flush_kernel<16, kFlushRowsFew, OUT><<<grid, wg, 0, s>>>(S, pv, pr, m, q, g, x, ymu, out, N, D, A);
+    else
+        decode_flush_kernel<16, kFlushRows, OUT><<<grid, wg, 0, s>>>(S, pv, pr, m, q, g, x, ymu, out, N, D, A);
+    return check_launch("decode_flush_kernel");
+}
+}  // namespace
+
+// S_base <- S_t with its m pending terms, and nothing read out (S and pr
+// 16-byte aligned, A % 4 == 0, A <= 4096: checked by the caller)
+int launch_decode_write_back(float *S, const float *pv, const float *pr, int m, const float *g, int N, int D, int A,
+                             hipStream_t s) {
+    return launch_flush<false>(S, pv, pr, m, nullptr, g, nullptr, nullptr, nullptr, N, D, A, s);
 }
 
 }  // namespace ulm
@@ -531,14 +567,7 @@ extern "C" int ulm_decode_flush(float *S, const float *pv, const float *pr, int 
                 A);
     ULM_REQUIRE(S && pv && pr && q && g && x && ymu && out, "ulm_decode_flush: null pointer");
     ULM_REQUIRE(aligned16({S, q, pr}), "ulm_decode_flush: S, q and the pending keys must be 16-byte aligned");
-    const int waves = (A / 4 + kWave - 1) / kWave;   // one 256-slot strip per wave
-    const dim3 grid(N, (D + kFlushRows - 1) / kFlushRows);
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    if (waves <= 12)
-        decode_flush_kernel<12><<<grid, dim3(waves * kWave), 0, s>>>(S, pv, pr, m, q, g, x, ymu, out, N, D, A);
-    else
-        decode_flush_kernel<16><<<grid, dim3(waves * kWave), 0, s>>>(S, pv, pr, m, q, g, x, ymu, out, N, D, A);
-    return check_launch("decode_flush_kernel");
+    return launch_flush<true>(S, pv, pr, m, q, g, x, ymu, out, N, D, A, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int ulm_decode_addr_deferred(const float *pre, const float *bias, const float *log_eps, const float *w,

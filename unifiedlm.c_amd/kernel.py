@@ -16,6 +16,7 @@ Besides the operator this module exposes the relu^2 slot address
 (model.py:70-72) as an autograd Function and the three per-token decode
 kernels used by UnifiedBlock.step.
 """
+import struct
 from typing import Optional
 
 import torch
@@ -719,6 +720,56 @@ def decode_addr_deferred(pre, bias, log_eps, w, g, r_prev, c, pr, slot, dots):
          ptr(_f32c(w)), ptr(_f32c(g)), ptr(_f32c(r_prev)), ptr(_f32c(c)), ptr(r), ptr(q), ptr(wq), ptr(_f32c(pr)),
          slot, ptr(cj), N, A, nat.stream_of(pre))
     return r, q, wq, cj
+
+
+# the tensors of one layer of ulm_decode_step, in the order of its struct
+_STEP_PARAMS = ("norm_w", "conv_w", "key_w", "key_b", "log_eps", "val_w", "mu_w", "w", "g")
+_STEP_STATE = ("buf", "S", "c", "r_prev", "pv", "pr")
+_STEP_ALIGNED = 1 << 6 | 1 << 7 | 1 << 10 | 1 << 11 | 1 << 12   # mu_w, w, S, c, r_prev: 16-byte accesses
+
+
+def decode_step(x, states, norm_eps):
+    """One position of consecutive blocks in two launches
+    per block (ulm_decode_step): x (N, D) fp32, states the blocks' deferred
+    decode states (dicts of _STEP_STATE, the pending count "np" and the
+    parameters "params"), norm_eps their norms' epsilons. The states are
+    updated in place. Returns the last block's output, or None, with nothing
+    touched, for a call this form does not take (large states, other dtypes or
+    layouts, tensors that disagree with each other): the per-kernel
+    form serves those, or refuses them."""
+    if x.dim() != 2 or x.dtype != torch.float32 or not x.is_cuda or not x.is_contiguous():
+        return None
+    N, D = x.shape
+    if states[0]["S"].dim() != 3 or states[0]["params"]["conv_w"].dim() != 2:
+        return None
+    A, Kc = states[0]["S"].shape[2], states[0]["params"]["conv_w"].shape[1]
+    ws_bytes = nat.lib().ulm_decode_step_workspace_bytes(N, D, A, Kc)
+    if ws_bytes == 0:
+        return None
+    dev = x.get_device()
+    J = 16
+    shapes = ((D,), (D, Kc), (A, D), (A,), (1,), (D, D), (D, A), (A,), (1,),
+              (N, D, Kc - 1), (N, D, A), (N, A), (N, A), (J, N, D), (J, N, A))
+    fields = []
+    for s, eps in zip(states, norm_eps):
+        p = s["params"]
+        for i, t in enumerate([p[k] for k in _STEP_PARAMS] + [s[k] for k in _STEP_STATE]):
+            if (t.shape != shapes[i] or t.dtype != torch.float32 or t.get_device() != dev or not t.is_contiguous()):
+                return None
+            at = t.data_ptr()
+            if at & 15 and _STEP_ALIGNED >> i & 1:
+                return None
+            fields.append(at)
+        if not 0 <= s["np"] < J:
+            return None
+        fields += (eps, s["np"])
+    layers = struct.pack("@" + "15Pdq" * len(states), *fields)
+    out = torch.empty_like(x)
+    ws = torch.empty(ws_bytes, device=x.device, dtype=torch.uint8)
+    call("ulm_decode_step", layers, len(states), ptr(x), ptr(out), ptr(ws), ws_bytes, N, D, A, Kc, nat.stream_of(x))
+    for s in states:
+        s["np"] = (s["np"] + 1) % J
+    return out
 
 
 def decode_deferred(S, pv, pr, m, flush, q, g, x, ymu, cj=None):

@@ -30,7 +30,7 @@ import torch.nn.functional as F
 
 from kernel import (CHUNK, LOG_W_MAX, LOG_W_MIN, block_prefill, decode_addr, decode_addr_deferred, decode_deferred,
                     decode_pre, decode_state,
-                    fm_prefill,
+                    decode_step, fm_prefill,
                     relu2_address, unified_block, unified_memory)
 
 
@@ -149,15 +149,15 @@ class UnifiedBlock(nn.Module):
 
     @torch.no_grad()
     def _step_params(self, device):
-        """fp32 copies of what every step reads, in the layouts of the decode
-        kernels (taken once per decode session: weights do not change while it
-        decodes)."""
+        """What every step reads, in contiguous fp32 (the parameters themselves
+        where they are that already), taken once per decode session: weights
+        do not change while it decodes."""
         def f32(t):
             return t.detach().to(device=device, dtype=torch.float32).contiguous()
         return {"norm_w": f32(self.norm.weight), "conv_w": f32(self.conv.weight[:, 0, :]),
-                "key_wt": f32(self.key.weight.t()), "key_b": f32(self.key.bias),
-                "log_eps": f32(self.log_eps).reshape(1), "val_wt": f32(self.val.weight.t()),
-                "mu_wt": f32(self.mu.weight.t()), "w": f32(self._w()), "g": f32(self._decay_log()).reshape(1)}
+                "key_w": f32(self.key.weight), "key_b": f32(self.key.bias),
+                "log_eps": f32(self.log_eps).reshape(1), "val_w": f32(self.val.weight),
+                "mu_w": f32(self.mu.weight), "w": f32(self._w()), "g": f32(self._decay_log()).reshape(1)}
 
     @torch.no_grad()
     def init_state(self, batch: int, device):
@@ -200,6 +200,15 @@ class UnifiedBlock(nn.Module):
             buf[:, :, kw - n:] = h[:, T - n:, :].float().transpose(1, 2)
         return out, {"buf": buf, "S": S, "c": c, "r_prev": r_prev, "params": self._step_params(x.device)}
 
+    @staticmethod
+    def _pending(s, device):
+        """A deferred state's room for its pending terms, made at its first step."""
+        if "pv" not in s:
+            N, width, slots = s["S"].shape
+            s["pv"] = torch.empty(DECODE_PENDING, N, width, device=device, dtype=torch.float32)
+            s["pr"] = torch.empty(DECODE_PENDING, N, slots, device=device, dtype=torch.float32)
+            s["np"] = 0
+
     @torch.no_grad()
     def step(self, x, s):
         """One position x (B, d) for a batch of sequences: write (key r_{t-1},
@@ -211,26 +220,30 @@ class UnifiedBlock(nn.Module):
         appends its term and reads S with the terms added, and the position
         that fills the last term writes S back with all of them. The maths of
         model.py:107-109 in another order: S moves one write per
-        DECODE_PENDING positions instead of one per position."""
+        DECODE_PENDING positions instead of one per position. A small
+        batch of it takes two launches in all (kernel.decode_step)."""
         p = s["params"]
         x32 = x.float().contiguous()
-        h, u = decode_pre(x32, p["norm_w"], p["conv_w"], s["buf"], self.norm.eps)
         N, width, slots = s["S"].shape
-        if slots % 4 or slots > 4096:
-            r, q, wq = decode_addr(u @ p["key_wt"], p["key_b"], p["log_eps"], p["w"], p["g"], s["r_prev"], s["c"])
-            out = decode_state(s["S"], h @ p["val_wt"], s["r_prev"], q, p["g"], x32, wq @ p["mu_wt"])
+        deferred = slots % 4 == 0 and slots <= 4096
+        if deferred:
+            self._pending(s, x.device)
+            out = _few_step(x32, [self], [s])
+            if out is not None:
+                return out.to(x.dtype)
+        h, u = decode_pre(x32, p["norm_w"], p["conv_w"], s["buf"], self.norm.eps)
+        pre = F.linear(u, p["key_w"])
+        if not deferred:
+            r, q, wq = decode_addr(pre, p["key_b"], p["log_eps"], p["w"], p["g"], s["r_prev"], s["c"])
+            out = decode_state(s["S"], F.linear(h, p["val_w"]), s["r_prev"], q, p["g"], x32, F.linear(wq, p["mu_w"]))
         else:
-            if "pv" not in s:
-                s["pv"] = torch.empty(DECODE_PENDING, N, width, device=x.device, dtype=torch.float32)
-                s["pr"] = torch.empty(DECODE_PENDING, N, slots, device=x.device, dtype=torch.float32)
-                s["np"] = 0
             m = s["np"]
             flush = m + 1 == DECODE_PENDING
             # appends r_prev as pending key m (and the terms' read-out weights unless this position writes back)
-            r, q, wq, cj = decode_addr_deferred(u @ p["key_wt"], p["key_b"], p["log_eps"], p["w"], p["g"],
-                                                s["r_prev"], s["c"], s["pr"], m, not flush)
-            torch.mm(h, p["val_wt"], out=s["pv"][m])
-            out = decode_deferred(s["S"], s["pv"], s["pr"], m + 1, flush, q, p["g"], x32, wq @ p["mu_wt"], cj)
+            r, q, wq, cj = decode_addr_deferred(pre, p["key_b"], p["log_eps"], p["w"], p["g"], s["r_prev"], s["c"],
+                                                s["pr"], m, not flush)
+            torch.mm(h, p["val_w"].t(), out=s["pv"][m])
+            out = decode_deferred(s["S"], s["pv"], s["pr"], m + 1, flush, q, p["g"], x32, F.linear(wq, p["mu_w"]), cj)
             s["np"] = 0 if flush else m + 1
         s["r_prev"] = r
         return out.to(x.dtype)
@@ -250,6 +263,15 @@ class UnifiedBlock(nn.Module):
         decode_deferred(s["S"], s["pv"], s["pr"], m, True, zeros, p["g"], x0, x0)   # the read-out is discarded
         s["np"] = 0
         return s
+
+
+def _few_step(x, layers, states):
+    """kernel.decode_step over consecutive UnifiedBlocks, or None where it does
+    not apply. Under autocast the projections of the per-kernel form are
+    autocast's, so that form keeps such calls."""
+    if torch.is_autocast_enabled("cuda"):
+        return None
+    return decode_step(x, states, [layer.norm.eps for layer in layers])
 
 
 class UnifiedLM(nn.Module):
@@ -327,9 +349,28 @@ class UnifiedLM(nn.Module):
     def step(self, tokens: torch.Tensor, states) -> torch.Tensor:
         """One position for a batch of sequences: tokens (B,) -> logits (B, V)."""
         h = self.tok_embeddings(tokens)
+        out = self._few_steps(h, states)
+        if out is None:
+            for layer, s in zip(self.layers, states):
+                h = layer.step(h, s)
+            out = h
+        return self.output(self.norm(out))
+
+    def _few_steps(self, h, states):
+        """Every block's step in one native call (kernel.decode_step), or None
+        where a block would not take it by itself: other dtypes, large states,
+        slot counts without the deferred state, steps of a
+        subclass's own."""
+        if h.dtype != torch.float32 or len(states) != len(self.layers):
+            return None
         for layer, s in zip(self.layers, states):
-            h = layer.step(h, s)
-        return self.output(self.norm(h))
+            if type(layer) is not UnifiedBlock or "step" in layer.__dict__:
+                return None
+            slots = s["S"].shape[-1]
+            if slots % 4 or slots > 4096:
+                return None
+            layer._pending(s, h.device)
+        return _few_step(h, self.layers, states) if states else None
 
     @torch.no_grad()
     def decode_greedy(self, prompt: torch.Tensor, steps: int, prefill: bool = True) -> torch.Tensor:

@@ -59,6 +59,8 @@ SIGNATURES = {
     "ulm_decode_dots": (I, [P, P, P, I, I, I, P]),
     "ulm_decode_read": (I, [P, P, P, I, P, P, P, P, P, I, I, I, P]),
     "ulm_decode_flush": (I, [P, P, P, I, P, P, P, P, P, I, I, I, P]),
+    "ulm_decode_step_workspace_bytes": (SZ, [I, I, I, I]),
+    "ulm_decode_step": (I, [P, I, P, P, P, SZ, I, I, I, I, P]),
     "ulm_la_timer_start": (I, [I]),
     "ulm_la_timer_stop": (I, [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int)]),
     "ulm_la_timer_product": (I, [I, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int)]),
