@@ -1,0 +1,135 @@
+"""The host module's eager calls (csrc/host.cpp) against the registered ops and
+the Python implementations they stand in for, bit for bit, and the calls that
+it leaves to those (needs an MI355X)."""
+import pytest
+import torch
+
+from helpers import say
+
+pytestmark = pytest.mark.gpu
+
+import kernel  # noqa: E402
+import ulm_native as nat  # noqa: E402
+from model import ModelArgs, UnifiedBlock  # noqa: E402
+
+
+def _args(B, T, D, A, taps, seed, form="plain", bias=True):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    rn = lambda *s, std=1.0: torch.randn(*s, device="cuda", generator=gen) * std  # noqa: E731
+    x = rn(B, T, D)
+    key = rn(A, D, std=D ** -0.5)
+    if form == "strided":   # an input and a weight that are views in another order
+        x, key = rn(T, B, D).transpose(0, 1), rn(D, A, std=D ** -0.5).t()
+    if form == "half":      # weights kept in bf16
+        key = key.to(torch.bfloat16)
+    t = [x, 1 + rn(D, std=0.1), rn(D, 1, taps, std=0.5), key, rn(A, std=0.1) if bias else None,
+         torch.zeros((), device="cuda"), rn(D, D, std=D ** -0.5), rn(D, A, std=0.05), torch.tensor(-3.0, device="cuda"),
+         rn(A, std=0.4)]
+    return [None if a is None else a.detach().requires_grad_(True) for a in t], rn(B, T, D)
+
+
+BLOCKS = [(2, 70, 64, 96, 4, "plain", True), (1, 1, 7, 5, 1, "plain", True), (3, 130, 40, 70, 8, "strided", True),
+          (2, 33, 96, 128, 3, "plain", False), (2, 200, 288, 712, 4, "half", True)]
+
+
+@pytest.mark.parametrize("cdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,T,D,A,taps,form,bias", BLOCKS)
+def test_block_equals_registered_op(B, T, D, A, taps, form, bias, cdt):
+    say(f"host block vs registered op B={B} T={T} D={D} A={A} taps={taps} {form} {cdt}")
+    args, dout = _args(B, T, D, A, taps, T + D, form, bias)
+    leaves = [a for a in args if a is not None]
+    got = kernel.block_eager(*args, 1e-5, cdt)
+    assert got is not None
+    g1 = torch.autograd.grad(got, leaves, dout)
+    ref = kernel.block_fwd(*args, 1e-5, cdt)[0]
+    g2 = torch.autograd.grad(ref, leaves, dout)
+    for a, b in zip((got, *g1), (ref, *g2)):
+        assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("cdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,T,D,A,taps,form,bias", BLOCKS)
+def test_prefill_equals_python(B, T, D, A, taps, form, bias, cdt):
+    say(f"host prefill vs block_prefill B={B} T={T} D={D} A={A} taps={taps} {form} {cdt}")
+    args, _ = _args(B, T, D, A, taps, T + D, form, bias)
+    out, S, c, r_prev, buf, g, w = kernel.block_prefill_eager(*args, 1e-5, cdt)
+    ref = kernel.block_prefill(*args, 1e-5, cdt)
+    for a, b in zip((out, S, c, r_prev), ref):
+        assert torch.equal(a, b)
+    n = min(taps - 1, T)
+    want = torch.zeros(B, D, taps - 1, device="cuda")
+    if n:
+        want[:, :, taps - 1 - n:] = ref[4][:, T - n:].float().transpose(1, 2)
+    assert torch.equal(buf, want) and not out.requires_grad
+    assert torch.equal(g[0], -torch.exp(args[8])) and torch.equal(w, torch.exp(args[9].clamp(-7, 12)))
+
+
+@pytest.mark.parametrize("which", ["both", "q", "fast"])
+def test_memory_equals_registered_op(which):
+    say(f"host unified_memory vs registered op, gradients of {which}")
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    r = torch.rand(2, 90, 70, device="cuda", generator=gen).to(torch.bfloat16) / 70
+    v = torch.randn(90, 2, 40, device="cuda", generator=gen).transpose(0, 1).to(torch.bfloat16)
+    g, w = torch.tensor(-0.05, device="cuda"), torch.full((70,), 4.0, device="cuda")
+    res = []
+    for host in (True, False):
+        leaves = [t.detach().clone().requires_grad_(True) for t in (r, v, g, w)]
+        out = nat.host().memory(*leaves) if host else kernel.fm_fwd(*leaves)[:2]
+        outs = {"both": out, "q": out[:1], "fast": out[1:]}[which]
+        grads = torch.autograd.grad(outs, leaves, [torch.ones_like(o) for o in outs])
+        res.append([*out, *grads])
+    for a, b in zip(*res):
+        assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b)
+
+
+def test_left_to_the_registered_ops():
+    say("calls the host module leaves alone")
+    args, _ = _args(2, 40, 32, 64, 4, 1)
+    host = nat.host()
+    take = lambda a, cdt=torch.float32: host.block(1e-5, cdt, *a)  # noqa: E731
+    assert take(args) is not None
+    swap = lambda i, t: args[:i] + [t] + args[i + 1:]  # noqa: E731
+    assert take(args, torch.float64) is None
+    assert take(swap(0, args[0].double())) is None and take(swap(0, args[0][0])) is None
+    assert take(swap(3, args[3].cpu())) is None and take(swap(9, args[9][:-1])) is None
+
+    class Sub(torch.Tensor):
+        pass
+    assert take(swap(0, args[0].detach().as_subclass(Sub))) is None
+    seen = []
+
+    def loss(x):
+        seen.append(take(swap(0, x)))
+        return kernel.block_fwd(x, *args[1:], 1e-5, torch.float32)[0].square().sum()
+    with pytest.raises(RuntimeError, match="functorch"):   # refused by the registered op, as without the host module
+        torch.func.grad(loss)(args[0].detach())
+    assert seen == [None]
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(args[0].detach(), torch.ones_like(args[0]))
+        assert take(swap(0, dual)) is None
+
+
+def test_saved_tensor_hooks_see_what_is_saved():
+    """Offloading hooks pack and unpack every tensor a block saves, inputs and intermediates."""
+    say("saved-tensor hooks over a block")
+    args, dout = _args(2, 40, 32, 64, 4, 1)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t.shape) or t.cpu(), lambda t: t.cuda()):
+        out = kernel.block_eager(*args, 1e-5, torch.float32)
+    assert len(packed) == 19
+    got = torch.autograd.grad(out, args, dout)
+    ref = torch.autograd.grad(kernel.block_eager(*args, 1e-5, torch.float32), args, dout)
+    assert all(torch.equal(a, b) for a, b in zip(got, ref))
+
+
+def test_module_forward_under_autocast():
+    say("UnifiedBlock.forward: the autocast dtype reaches the host path")
+    torch.manual_seed(0)
+    block = UnifiedBlock(ModelArgs(dim=64, hidden_dim=96)).cuda()
+    x = torch.randn(2, 50, 64, device="cuda")
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        got = block(x)
+    p = block
+    ref = kernel.block_fwd(x, p.norm.weight, p.conv.weight, p.key.weight, p.key.bias, p.log_eps, p.val.weight,
+                           p.mu.weight, p.log_rate, p.log_w, p.norm.eps, torch.bfloat16)[0]
+    assert torch.equal(got, ref) and got.requires_grad

@@ -4,7 +4,8 @@
 
 Every source under csrc/ is compiled for gfx950 by hipcc into _build/ and
 linked into unifiedlm.c_amd/libulm_fm.so, next to the Python modules that load
-it; the layout probes (probe.hip) go into a test-only libulm_probe.so beside it. Packed fp32 VALU instructions are disabled (-packed-fp32-ops) and fp32
+it; the layout probes (probe.hip) go into a test-only libulm_probe.so beside it, and
+the host module (host.cpp, C++ against torch) into ulm_host.so. Packed fp32 VALU instructions are disabled (-packed-fp32-ops) and fp32
 atomics use the hardware add (-munsafe-fp-atomics).
 """
 import concurrent.futures
@@ -18,6 +19,7 @@ CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libulm_fm.so")
 PROBE_LIB = os.path.join(HERE, "libulm_probe.so")
+HOST_LIB = os.path.join(HERE, "ulm_host.so")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 
 SOURCES = ["status.hip", "elementwise.hip", "decode.hip", "decode_step.hip", "address.hip", "fm_stats.hip", "fm_chunk.hip", "pair.hip",
@@ -62,17 +64,50 @@ def _link(objs, lib):
     os.replace(tmp, lib)
 
 
+def _build_host():
+    """The host module (host.cpp, no GPU code) against torch and libulm_fm.so,
+    which it finds beside itself. Returns the compiler's warnings."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    obj = os.path.join(BUILD, "host.o")
+    incs = cpp_extension.include_paths() + [sysconfig.get_paths()["include"], "/opt/rocm/include", INCLUDE]
+    cmd = ["g++", "-O2", "-fPIC", "-std=c++17", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    cmd += [f"-isystem{p}" for p in incs] + ["-c", os.path.join(CSRC, "host.cpp"), "-o", obj]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on host.cpp:\n{res.stderr}")
+    return res.stderr
+
+
+def _link_host():
+    from torch.utils import cpp_extension
+    tmp = HOST_LIB + ".tmp"
+    cmd = ["g++", "-shared", "-o", tmp, os.path.join(BUILD, "host.o"), f"-L{HERE}", "-lulm_fm", "-Wl,-rpath,$ORIGIN"]
+    cmd += [f"-L{p}" for p in cpp_extension.library_paths()]
+    cmd += ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"link of ulm_host.so failed:\n{res.stderr}")
+    os.replace(tmp, HOST_LIB)
+
+
 def build(verbose=False):
-    """Compile every source and link both shared libraries (always rebuilds)."""
+    """Compile every source and link the shared libraries (always rebuilds)."""
     os.makedirs(BUILD, exist_ok=True)
     sources = sorted(set(SOURCES) | set(PROBE_SOURCES))
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(sources))) as ex:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(sources) + 1)) as ex:
+        host = ex.submit(_build_host)
         results = dict(zip(sources, ex.map(_compile, sources)))
     for obj, err in results.values():
         if err and verbose:
             print(err, file=sys.stderr)
     _link([results[src][0] for src in SOURCES], LIB)
     _link([results[src][0] for src in PROBE_SOURCES], PROBE_LIB)
+    host.result()
+    _link_host()
     return LIB
 
 

@@ -16,7 +16,6 @@ Besides the operator this module exposes the relu^2 slot address
 (model.py:70-72) as an autograd Function and the three per-token decode
 kernels used by UnifiedBlock.step.
 """
-import struct
 from typing import Optional
 
 import torch
@@ -138,18 +137,14 @@ def _fm_setup(ctx, inputs, output):
     ctx.set_materialize_grads(False)
 
 
-def _fm_backward_with(bwd, ctx, dq_out, dfast):
+def _fm_backward(ctx, dq_out, dfast, _dsaved):
     r, g, w, saved = ctx.saved_tensors
     if dq_out is None and dfast is None:
         return None, None, None, None
     if dfast is None:
         dfast = r.new_zeros(*r.shape[:2], ctx.D, dtype=torch.float32)
-    dr, dv, dg, dw = bwd(r, g, w, saved, ctx.v_dtype, dq_out, dfast)
+    dr, dv, dg, dw = fm_bwd(r, g, w, saved, ctx.v_dtype, dq_out, dfast)
     return dr, dv, dg.reshape(g.shape), dw
-
-
-def _fm_backward(ctx, dq_out, dfast, _dsaved):
-    return _fm_backward_with(fm_bwd, ctx, dq_out, dfast)
 
 
 torch.library.register_autograd("ulm::fm_fwd", _fm_backward, setup_context=_fm_setup)
@@ -161,39 +156,24 @@ _dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", lambda: 1)
 
 def _plain_eager(*tensors):
     """True when the call runs eagerly on plain tensors: no torch.compile
-    trace, no dispatch mode (fake tensors, functionalization) and no tensor
-    subclass, so the native kernels can be called without the registered
-    op's dispatch."""
+    trace, no dispatch mode (fake tensors, functionalization), and tensors or
+    parameters proper. The host module then takes it, without the registered
+    ops' dispatch and Python between the launches; the registered ops serve
+    the rest (the module itself looks at the tensors it is given)."""
     if torch.compiler.is_compiling() or _dispatch_modes() > 0:
         return False
-    return all(type(t) is torch.Tensor for t in tensors)
-
-
-class _FMEager(torch.autograd.Function):
-    """The registered op pair ulm::fm_fwd / ulm::fm_bwd as a plain autograd
-    Function over the same implementations: the eager path, without the
-    registered ops' dispatch (about 20 us of host time per call, which
-    small shapes feel). torch.compile traces the registered ops instead."""
-
-    @staticmethod
-    def forward(ctx, r, v, g, w):
-        out = _fm_fwd_impl(r, v, g, w)
-        _fm_setup(ctx, (r, v, g, w), out)
-        return out
-
-    @staticmethod
-    def backward(ctx, dq_out, dfast, _dsaved):
-        return _fm_backward_with(_fm_bwd_impl, ctx, dq_out, dfast)
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
 
 
 def unified_memory(r, v, g, w):
     """r: (B,T,M) read addresses, v: (B,T,D) values, g: scalar log decay, w: (M,) prior mass.
     Returns (q fp32, fast in v's dtype) (kernel.py:236-238)."""
+    if _plain_eager():
+        out = nat.host().memory(r, v, g, w)
+        if out is not None:
+            return out
     _check_fm(r, v, g, w)
-    if _plain_eager(r, v, g, w):
-        q, fast, _ = _FMEager.apply(r, v, g, w)
-    else:
-        q, fast, _ = fm_fwd(r, v, g, w)
+    q, fast, _ = fm_fwd(r, v, g, w)
     return q, fast
 
 
@@ -548,6 +528,13 @@ def _block_backward(ctx, dout, *_unused):
 torch.library.register_autograd("ulm::block_fwd", _block_backward, setup_context=_block_setup)
 
 
+def block_eager(x, norm_w, conv_w, key_w, key_b, log_eps, val_w, mu_w, log_rate, log_w, norm_eps, cdt):
+    """unified_block of a plain eager call on the host module, or None."""
+    if not _plain_eager():
+        return None
+    return nat.host().block(norm_eps, cdt, x, norm_w, conv_w, key_w, key_b, log_eps, val_w, mu_w, log_rate, log_w)
+
+
 def unified_block(x, norm_w, conv_w, key_w, key_b, log_eps, val_w, mu_w, log_rate, log_w, norm_eps,
                   cdt=torch.float32):
     """x + mu(w q) + fast of one UnifiedBlock (model.py:77-85) in one fused
@@ -555,6 +542,9 @@ def unified_block(x, norm_w, conv_w, key_w, key_b, log_eps, val_w, mu_w, log_rat
     val_w (D, D), conv_w (D, 1, Kc); log_rate (a scalar) and log_w (A,) are the
     block's parameters: g = -exp(log_rate), w = exp(clamp(log_w, LOG_W_MIN,
     LOG_W_MAX)) (model.py:75, 84) are formed, and differentiated, natively."""
+    out = block_eager(x, norm_w, conv_w, key_w, key_b, log_eps, val_w, mu_w, log_rate, log_w, float(norm_eps), cdt)
+    if out is not None:
+        return out
     if x.dim() != 3 or x.dtype != torch.float32:
         raise ValueError(f"x must be (B, T, D) fp32, got {tuple(x.shape)} {x.dtype}")
     B, T, D = x.shape
@@ -575,6 +565,14 @@ def unified_block(x, norm_w, conv_w, key_w, key_b, log_eps, val_w, mu_w, log_rat
 
 # ---------------------------------------------------------------------------
 # per-token decode (model.py:96-111), N sequences at once, fp32
+
+def block_prefill_eager(x, norm_w, conv_w, key_w, key_b, log_eps, val_w, mu_w, log_rate, log_w, norm_eps, cdt):
+    """block_prefill of a plain eager call on the host module, or None: (out,
+    S, c, r_prev, the conv window (B, D, taps - 1) fp32, g, w)."""
+    if not _plain_eager():
+        return None
+    return nat.host().prefill(norm_eps, cdt, x, norm_w, conv_w, key_w, key_b, log_eps, val_w, mu_w, log_rate, log_w)
+
 
 @torch.no_grad()
 def block_prefill(x, norm_w, conv_w, key_w, key_b, log_eps, val_w, mu_w, log_rate, log_w, norm_eps,
@@ -722,54 +720,16 @@ def decode_addr_deferred(pre, bias, log_eps, w, g, r_prev, c, pr, slot, dots):
     return r, q, wq, cj
 
 
-# the tensors of one layer of ulm_decode_step, in the order of its struct
-_STEP_PARAMS = ("norm_w", "conv_w", "key_w", "key_b", "log_eps", "val_w", "mu_w", "w", "g")
-_STEP_STATE = ("buf", "S", "c", "r_prev", "pv", "pr")
-_STEP_ALIGNED = 1 << 6 | 1 << 7 | 1 << 10 | 1 << 11 | 1 << 12   # mu_w, w, S, c, r_prev: 16-byte accesses
-
-
 def decode_step(x, states, norm_eps):
     """One position of consecutive blocks in two launches
     per block (ulm_decode_step): x (N, D) fp32, states the blocks' deferred
-    decode states (dicts of _STEP_STATE, the pending count "np" and the
-    parameters "params"), norm_eps their norms' epsilons. The states are
-    updated in place. Returns the last block's output, or None, with nothing
-    touched, for a call this form does not take (large states, other dtypes or
-    layouts, tensors that disagree with each other): the per-kernel
-    form serves those, or refuses them."""
-    if x.dim() != 2 or x.dtype != torch.float32 or not x.is_cuda or not x.is_contiguous():
-        return None
-    N, D = x.shape
-    if states[0]["S"].dim() != 3 or states[0]["params"]["conv_w"].dim() != 2:
-        return None
-    A, Kc = states[0]["S"].shape[2], states[0]["params"]["conv_w"].shape[1]
-    ws_bytes = nat.lib().ulm_decode_step_workspace_bytes(N, D, A, Kc)
-    if ws_bytes == 0:
-        return None
-    dev = x.get_device()
-    J = 16
-    shapes = ((D,), (D, Kc), (A, D), (A,), (1,), (D, D), (D, A), (A,), (1,),
-              (N, D, Kc - 1), (N, D, A), (N, A), (N, A), (J, N, D), (J, N, A))
-    fields = []
-    for s, eps in zip(states, norm_eps):
-        p = s["params"]
-        for i, t in enumerate([p[k] for k in _STEP_PARAMS] + [s[k] for k in _STEP_STATE]):
-            if (t.shape != shapes[i] or t.dtype != torch.float32 or t.get_device() != dev or not t.is_contiguous()):
-                return None
-            at = t.data_ptr()
-            if at & 15 and _STEP_ALIGNED >> i & 1:
-                return None
-            fields.append(at)
-        if not 0 <= s["np"] < J:
-            return None
-        fields += (eps, s["np"])
-    layers = struct.pack("@" + "15Pdq" * len(states), *fields)
-    out = torch.empty_like(x)
-    ws = torch.empty(ws_bytes, device=x.device, dtype=torch.uint8)
-    call("ulm_decode_step", layers, len(states), ptr(x), ptr(out), ptr(ws), ws_bytes, N, D, A, Kc, nat.stream_of(x))
-    for s in states:
-        s["np"] = (s["np"] + 1) % J
-    return out
+    decode states (dicts of buf, S, c, r_prev, pv and pr, the pending count
+    "np" and the parameters "params"), norm_eps their norms' epsilons. The
+    states are updated in place. Returns the last block's output, or None,
+    with nothing touched, for a call this form does not take (large states,
+    other dtypes or layouts, tensors that disagree with each other): the
+    per-kernel form serves those, or refuses them."""
+    return nat.host().decode_step(x, states, norm_eps) if _plain_eager() else None
 
 
 def decode_deferred(S, pv, pr, m, flush, q, g, x, ymu, cj=None):

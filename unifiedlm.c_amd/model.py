@@ -28,9 +28,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from kernel import (CHUNK, LOG_W_MAX, LOG_W_MIN, block_prefill, decode_addr, decode_addr_deferred, decode_deferred,
-                    decode_pre, decode_state,
-                    decode_step, fm_prefill,
+from kernel import (CHUNK, LOG_W_MAX, LOG_W_MIN, block_eager, block_prefill, block_prefill_eager, decode_addr,
+                    decode_addr_deferred, decode_deferred, decode_pre, decode_state, decode_step, fm_prefill,
                     relu2_address, unified_block, unified_memory)
 
 
@@ -123,10 +122,13 @@ class UnifiedBlock(nn.Module):
         if x.dtype != torch.float32 or (self.training and self.dropout.p > 0):
             return self.forward_composed(x)
         cdt = _compute_dtype()
+        args = (x, self.norm.weight, self.conv.weight, self.key.weight, self.key.bias, self.log_eps, self.val.weight,
+                self.mu.weight, self.log_rate, self.log_w, self.norm.eps, cdt)
+        out = block_eager(*args)
+        if out is not None:
+            return out
         with torch.autocast("cuda", enabled=False):
-            return unified_block(x, self.norm.weight, self.conv.weight, self.key.weight, self.key.bias,
-                                 self.log_eps, self.val.weight, self.mu.weight, self.log_rate, self.log_w,
-                                 self.norm.eps, cdt)
+            return unified_block(*args)
 
     def _address_and_value(self, x):
         """h = RMSNorm(x), its causal depthwise conv u, the address r of u and
@@ -148,7 +150,7 @@ class UnifiedBlock(nn.Module):
     # ---- one position at a time (model.py:87-111)
 
     @torch.no_grad()
-    def _step_params(self, device):
+    def _step_params(self, device, w=None, g=None):
         """What every step reads, in contiguous fp32 (the parameters themselves
         where they are that already), taken once per decode session: weights
         do not change while it decodes."""
@@ -157,7 +159,8 @@ class UnifiedBlock(nn.Module):
         return {"norm_w": f32(self.norm.weight), "conv_w": f32(self.conv.weight[:, 0, :]),
                 "key_w": f32(self.key.weight), "key_b": f32(self.key.bias),
                 "log_eps": f32(self.log_eps).reshape(1), "val_w": f32(self.val.weight),
-                "mu_w": f32(self.mu.weight), "w": f32(self._w()), "g": f32(self._decay_log()).reshape(1)}
+                "mu_w": f32(self.mu.weight), "w": f32(self._w()) if w is None else w,
+                "g": f32(self._decay_log()).reshape(1) if g is None else g}
 
     @torch.no_grad()
     def init_state(self, batch: int, device):
@@ -182,6 +185,13 @@ class UnifiedBlock(nn.Module):
         B, T, width = x.shape
         if x.dtype == torch.float32:
             cdt = _compute_dtype()
+            done = block_prefill_eager(x, self.norm.weight, self.conv.weight, self.key.weight, self.key.bias,
+                                       self.log_eps, self.val.weight, self.mu.weight, self.log_rate, self.log_w,
+                                       self.norm.eps, cdt)
+            if done is not None:
+                out, S, c, r_prev, buf, g, w = done
+                return out, {"buf": buf, "S": S, "c": c, "r_prev": r_prev,
+                             "params": self._step_params(x.device, w, g)}
             with torch.autocast("cuda", enabled=False):
                 out, S, c, r_prev, h = block_prefill(x, self.norm.weight, self.conv.weight, self.key.weight,
                                                      self.key.bias, self.log_eps, self.val.weight, self.mu.weight,

@@ -113,6 +113,23 @@ def lib():
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The host module (csrc/host.cpp); raises if it was never built."""
+    global _host
+    if _host is None:
+        lib()   # the library it is linked against
+        try:
+            import ulm_host
+        except ImportError as e:
+            raise RuntimeError(f"ulm_host.so cannot be loaded from {HERE} ({e}): build it with "
+                               "`python unifiedlm.c_amd/build.py`") from e
+        _host = ulm_host
+    return _host
+
+
 def call(name, *args):
     """Calls an entry point and raises RuntimeError on a nonzero status."""
     status = getattr(lib(), name)(*args)
