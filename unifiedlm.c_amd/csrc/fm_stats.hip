@@ -67,6 +67,7 @@ struct RTensor {
     __device__ __forceinline__ float slot_const(int) const { return 0.f; }
     static constexpr bool kRowConst = false;
     __device__ __forceinline__ float row_raw(size_t, bool) const { return 1.f; }
+    __device__ __forceinline__ const raw_t *rows(size_t row, int A) const { return r + row * A; }
     __device__ __forceinline__ raw_t raw(size_t row, uint32_t ac, int A) const { return ld_row(r + row * A, 4u * ac); }
     __device__ __forceinline__ float make(raw_t v, float, float, bool ok) const { return ok ? v : 0.f; }
     __device__ __forceinline__ float at(size_t row, uint32_t ac, int A, float b, float inv, bool ok) const {
@@ -90,6 +91,7 @@ struct RAddr {
     __device__ __forceinline__ float slot_const(int a) const { return bias ? bias[a] : 0.f; }
     static constexpr bool kRowConst = true;
     __device__ __forceinline__ float row_raw(size_t row, bool tok) const { return denom[tok ? row : 0]; }
+    __device__ __forceinline__ const raw_t *rows(size_t row, int A) const { return pre + row * A; }
     __device__ __forceinline__ raw_t raw(size_t row, uint32_t ac, int A) const {
         return ld_row(pre + row * A, static_cast<uint32_t>(sizeof(TP)) * ac);
     }
@@ -125,6 +127,34 @@ template <class RS> __device__ __forceinline__ float seg_inv(float d) {
 
 __device__ __forceinline__ float lane_value(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// Range-checked buffers: reads past the range give zeros, writes are dropped. A
+// lane whose offset carries kOut is always past it.
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+constexpr uint32_t kOut = 0x80000000u;
+// base and bytes are wave-uniform; the compiler is told so, or it would walk the lanes' descriptors in a loop
+__device__ __forceinline__ rsrc_t make_rsrc(const void *base, uint32_t bytes) {
+    const uint64_t p = reinterpret_cast<uint64_t>(base);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p));
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(p >> 32));
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void *>(static_cast<uint64_t>(hi) << 32 | lo), 0,
+                                             __builtin_amdgcn_readfirstlane(static_cast<int>(bytes)), 0x00020000);
+}
+template <class E> __device__ __forceinline__ E buf_load(rsrc_t r, uint32_t off) {
+    if constexpr (sizeof(E) == 4) return __builtin_bit_cast(E, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+    else return __builtin_bit_cast(E, static_cast<uint16_t>(__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0)));
+}
+template <class E> __device__ __forceinline__ void buf_store(E v, rsrc_t r, uint32_t off) {
+    if constexpr (sizeof(E) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, off, 0, 0);
+    else __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, v), r, off, 0, 0);
+}
+
+// num / den to within an ulp, from den's reciprocal and one correction, for
+// normal den; zeros, infinities and NaN as a division has them
+__device__ __forceinline__ float quotient(float num, float den) {
+    const float rc = __builtin_amdgcn_rcpf(den), q0 = num * rc;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-den, q0, num), rc, q0), den, num);
 }
 
 // Row b T + t of a (B, T, ...) tensor when 0 <= t < T, else row 0: the clamp
@@ -196,8 +226,16 @@ __global__ __launch_bounds__(1024) void fwd_segtot_kernel(RS rs, const float *__
 // decode state as one product over positions).
 // segtot: the segment totals of sequences past one segment (see above).
 // QW: the dtype of the w q output (-1 none, else a ulm_dtype); HAS_Q: the fp32 q output.
-template <class RS, int QW, bool HAS_Q>
-__global__ __launch_bounds__(256) void fwd_stats_kernel(RS rs, const float *__restrict__ w,
+// CW: chunks walked side by side, 4 waves each. A sequence's chunks depend on
+// each other only through their 16-position segments' totals, so a walk over
+// few workgroups, which is bound by its latency, takes two at a time
+// (launch_fwd_stats). Every thread folds the totals before it in the same
+// order either way, so CW does not change a bit.
+// At the 110M training shape (768 workgroups) the kernel is bound by its
+// 805 MB: 139 us with r and q in fp32 (5.8 TB/s; 165 before its instructions
+// were cut, see the walk below), 110 us in the fused block (147).
+template <class RS, int QW, bool HAS_Q, int CW>
+__global__ __launch_bounds__(256 * CW, 3) void fwd_stats_kernel(RS rs, const float *__restrict__ w,
                                                         const float *__restrict__ g, float *__restrict__ q,
                                                         void *__restrict__ qw, int qw_dt,
                                                         uint16_t *__restrict__ q16n, uint16_t *__restrict__ k16n,
@@ -206,10 +244,14 @@ __global__ __launch_bounds__(256) void fwd_stats_kernel(RS rs, const float *__re
                                                         float *__restrict__ nck, float *__restrict__ c_last, int T,
                                                         int A, int AL, int NT, const float *__restrict__ segtot,
                                                         int S, int kq_decay) {
-    __shared__ float tot[4][kSlots];
-    __shared__ __align__(16) uint16_t sq[ULM_CHUNK][kSlots + 8], sk[ULM_CHUNK][kSlots + 8];   // [position][slot]
+    // [position][slot] of each of the CW chunks, q's then k's, then the 16-position segments' totals
+    using tile_t = uint16_t[ULM_CHUNK][kSlots + 8];
+    extern __shared__ __align__(16) char stats_lds[];
     const int s = threadIdx.x % kSlots;
-    const int j = __builtin_amdgcn_readfirstlane(threadIdx.x / kSlots);   // wave-uniform (kSlots = wave size)
+    const int js = __builtin_amdgcn_readfirstlane(threadIdx.x / kSlots);   // wave-uniform (kSlots = wave size)
+    const int j = js % 4, cw = js / 4;   // the 16-position segment of chunk cw of each group of CW chunks
+    tile_t &sq = reinterpret_cast<tile_t *>(stats_lds)[cw], &sk = reinterpret_cast<tile_t *>(stats_lds)[CW + cw];
+    float (*tot)[kSlots] = reinterpret_cast<float (*)[kSlots]>(stats_lds + 2 * CW * sizeof(tile_t));   // [4 CW]
     const int a0 = blockIdx.x * kSlots;
     const int a = a0 + s;
     const bool va = a < A;
@@ -230,27 +272,46 @@ __global__ __launch_bounds__(256) void fwd_stats_kernel(RS rs, const float *__re
         const float lamL = pow_2k(lam, 10);   // lam^1024, across one segment
         for (int i = 0; i < seg; ++i) carry = lamL * carry + (va ? segtot[(bs * S + i) * A + a] : 0.f);
     }
-    // the stored elements of a chunk's positions t0 .. t0+15 and t0 - 1, and
-    // their denominators, loaded two chunks ahead into alternating buffers
-    typename RS::raw_t pv[2][kSeg + 1];
+    // The stored elements of a chunk's positions t0 .. t0+15 and t0 - 1, and
+    // their denominators, loaded two groups ahead into alternating buffers. A
+    // chunk's rows are a range-checked buffer: positions past T and slots past A
+    // read as zero, and are not written, without a mask or a clamp.
+    using raw_t = typename RS::raw_t;
+    constexpr uint32_t es = sizeof(raw_t);
+    raw_t pv[2][kSeg + 1];
     float pd[2];
+    const uint32_t bad = va ? 0u : kOut;
+    const uint32_t off = (static_cast<uint32_t>(j * kSeg * A) + ac) | bad;   // elements from the chunk's first row
+    auto rows_of = [&](int n) { return static_cast<uint32_t>(max(min(ULM_CHUNK, T - n * ULM_CHUNK), 0)) * A; };
     auto fetch = [&](int n, int u) {
         const int t0 = n * ULM_CHUNK + j * kSeg;
         pd[u] = seg_row_raw(rs, bs * T + t0, t0, T, s);
+        const rsrc_t rows = make_rsrc(rs.rows(bs * T + n * ULM_CHUNK, A), es * rows_of(n));
+        pv[u][kSeg] = ld_row(rs.rows(bs * T + min(max(t0 - 1, 0), T - 1), A), es * ac);
 #pragma unroll
-        for (int i = 0; i < kSeg; ++i) pv[u][i] = rs.raw(urow(bs, t0 + i, T), ac, A);
-        pv[u][kSeg] = rs.raw(urow(bs, t0 - 1, T), ac, A);
+        for (int i = 0; i < kSeg; ++i) pv[u][i] = buf_load<raw_t>(rows, es * (off + static_cast<uint32_t>(i * A)) | bad);
     };
-    fetch(n0, 0);
-    if (n0 + 1 < n1) fetch(n0 + 1, 1);
-    auto chunk = [&](int n, int u) {
+    fetch(n0 + cw, 0);
+    if (n0 + CW < n1) fetch(n0 + CW + cw, 1);
+    // chunk cw of the group that starts at chunk ng (past the segment's end:
+    // nothing written). The walk over the positions has no branch of its own:
+    // what few calls want (c at T - 1, decayed keys, natural copies) is done
+    // apart. Written with a mask, a clamp and those conditions at each position
+    // and in IEEE division steps, it took 169 instructions per position and
+    // slot, and a launch whose workgroups are few was bound by them.
+    auto group = [&](int ng, int u) {
+        const int n = ng + cw;
+        const bool on = n < n1;
         const int t0 = n * ULM_CHUNK + j * kSeg;
-        const float seg_c = seg_inv<RS>(pd[u]);
+        const int live = min(kSeg, T - t0);   // positions of this segment before T (may be negative)
+        // the positions' factors of r, 0 outside the sequence (lane l < 16: t0 + l, lane 16: t0 - 1)
+        float seg_c = seg_inv<RS>(pd[u]);
+        if constexpr (RS::kRowConst) seg_c = (s < kSeg ? s < live : t0 >= 1 && t0 <= T) ? seg_c : 0.f;
         float rv[kSeg], kv[kSeg], nl[kSeg];
 #pragma unroll
-        for (int i = 0; i < kSeg; ++i) rv[i] = rs.make(pv[u][i], rb, lane_value(seg_c, i), va && t0 + i < T);
+        for (int i = 0; i < kSeg; ++i) rv[i] = rs.make(pv[u][i], rb, lane_value(seg_c, i), true);
         kv[0] = rs.make(pv[u][kSeg], rb, lane_value(seg_c, kSeg), va && t0 >= 1 && t0 - 1 < T);
-        if (n + 2 < n1) fetch(n + 2, u);
+        if (ng + 2 * CW < n1) fetch(n + 2 * CW, u);
 #pragma unroll
         for (int i = 1; i < kSeg; ++i) kv[i] = rv[i - 1];
         float acc = 0.f;
@@ -259,46 +320,98 @@ __global__ __launch_bounds__(256) void fwd_stats_kernel(RS rs, const float *__re
             acc = lam * acc + kv[i];
             nl[i] = acc;
         }
-        tot[j][s] = acc;
+        tot[js][s] = acc;
         __syncthreads();
+        // n before this thread's segment: the group's earlier segments, in order
         float cj = carry;
-        for (int m = 0; m < j; ++m) cj = lam16 * cj + tot[m][s];
-        float pw = lam;
+        for (int m = 0; m < js; ++m) cj = lam16 * cj + tot[m][s];
+        float pw = lam, qt[kSeg], least = 3.0e38f;
         uint32_t qpk[kSeg / 2], kpk[kSeg / 2];   // bf16 pairs of this thread's 16 positions
 #pragma unroll
         for (int i = 0; i < kSeg; ++i) {
-            const int t = t0 + i;
-            const float ct = wa + (pw * cj + nl[i]);
+            nl[i] = wa + (pw * cj + nl[i]);   // c
             pw *= lam;
-            uint16_t qb = 0, kb = 0, kqb = 0;   // positions past T are zero in the tiled copies
-            if (va && t < T) {
-                const size_t ro = (bs * T + t) * A;   // wave-uniform row offset
-                const float qt = rv[i] / ct;
-                if (c_last && t == T - 1) c_last[bs * A + a] = ct;
-                qb = f32_to_bf16_bits(qt);
-                kb = f32_to_bf16_bits(kv[i]);
-                // kq_decay: the Q-layout keys decayed to T - 1, k_t lam^(T-1-t)
-                kqb = kq_decay ? f32_to_bf16_bits(kv[i] * __expf(lg * static_cast<float>(T - 1 - t))) : kb;
-                if constexpr (HAS_Q) st_row(q + ro, 4u * ac, qt);
-                if constexpr (QW == ULM_F32) st_row(static_cast<float *>(qw) + ro, 4u * ac, qt * wa);
-                if constexpr (QW == ULM_BF16) st_row(static_cast<uint16_t *>(qw) + ro, 2u * ac, f32_to_bf16_bits(qt * wa));
-                if constexpr (QW == ULM_F16) st_row(static_cast<_Float16 *>(qw) + ro, 2u * ac, static_cast<_Float16>(qt * wa));
-                if (q16n) {
-                    st_row(q16n + ro, 2u * ac, qb);
-                    st_row(k16n + ro, 2u * ac, kb);
-                }
-            }
-            sq[j * kSeg + i][s] = qb;
-            sk[j * kSeg + i][s] = kb;
-            if (i % 2 == 0) {
-                qpk[i / 2] = qb;
-                kpk[i / 2] = kqb;
-            } else {
-                qpk[i / 2] |= static_cast<uint32_t>(qb) << 16;
-                kpk[i / 2] |= static_cast<uint32_t>(kqb) << 16;
+            least = fminf(least, fabsf(nl[i]));
+        }
+        if (c_last && on && va && live > 0 && t0 + live == T) {
+            float cl = nl[0];
+#pragma unroll
+            for (int i = 1; i < kSeg; ++i) cl = i < live ? nl[i] : cl;
+            c_last[bs * A + a] = cl;
+        }
+        if (__any(least < 0x1p-120f)) {   // a prior mass next to nothing: its reciprocal may overflow
+#pragma unroll
+            for (int i = 0; i < kSeg; ++i) qt[i] = rv[i] / nl[i];
+        } else {
+#pragma unroll
+            for (int i = 0; i < kSeg; ++i) qt[i] = quotient(rv[i], nl[i]);
+        }
+        if (live < kSeg) {   // past T: zero in the copies (k at T is r at T - 1; q may be 0 / 0)
+#pragma unroll
+            for (int i = 0; i < kSeg; ++i) {
+                kv[i] = i < live ? kv[i] : 0.f;
+                qt[i] = i < live ? qt[i] : 0.f;
             }
         }
-        if ((qQ || kQ) && a < AL) {
+#pragma unroll
+        for (int i = 0; i < kSeg; i += 2) {
+            const bf16x2 qb = {static_cast<bf16>(qt[i]), static_cast<bf16>(qt[i + 1])};
+            const bf16x2 kb = {static_cast<bf16>(kv[i]), static_cast<bf16>(kv[i + 1])};
+            qpk[i / 2] = __builtin_bit_cast(uint32_t, qb);
+            kpk[i / 2] = __builtin_bit_cast(uint32_t, kb);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                sq[j * kSeg + i + e][s] = static_cast<uint16_t>(qpk[i / 2] >> (16 * e));
+                sk[j * kSeg + i + e][s] = static_cast<uint16_t>(kpk[i / 2] >> (16 * e));
+            }
+        }
+        const size_t row0 = (bs * T + n * ULM_CHUNK) * A;   // wave-uniform, of the chunk's first row
+        const uint32_t range = on ? rows_of(n) : 0u;        // elements of the chunk's rows
+        if constexpr (HAS_Q) {
+            const rsrc_t rq = make_rsrc(q + row0, 4u * range);
+#pragma unroll
+            for (int i = 0; i < kSeg; ++i) buf_store(qt[i], rq, 4u * (off + static_cast<uint32_t>(i * A)) | bad);
+        }
+        if constexpr (QW >= 0) {
+            using E = typename std::conditional<QW == ULM_F32, float,
+                                                typename std::conditional<QW == ULM_BF16, uint16_t, _Float16>::type>::type;
+            const rsrc_t rw = make_rsrc(static_cast<E *>(qw) + row0, static_cast<uint32_t>(sizeof(E)) * range);
+#pragma unroll
+            for (int i = 0; i < kSeg; ++i) {
+                E v;
+                if constexpr (QW == ULM_F32) v = qt[i] * wa;
+                if constexpr (QW == ULM_BF16) v = f32_to_bf16_bits(qt[i] * wa);
+                if constexpr (QW == ULM_F16) v = static_cast<_Float16>(qt[i] * wa);
+                buf_store(v, rw, static_cast<uint32_t>(sizeof(E)) * (off + static_cast<uint32_t>(i * A)) | bad);
+            }
+        }
+        if (va && on && live > 0) {
+            const size_t r0 = (bs * T + t0) * A;   // wave-uniform row offset
+            if (q16n) {
+#pragma unroll
+                for (int i = 0; i < kSeg; ++i) {
+                    if (i >= live) break;
+                    const size_t ro = r0 + static_cast<size_t>(i) * A;
+                    st_row(q16n + ro, 2u * ac, static_cast<uint16_t>(qpk[i / 2] >> (16 * (i % 2))));
+                    st_row(k16n + ro, 2u * ac, static_cast<uint16_t>(kpk[i / 2] >> (16 * (i % 2))));
+                }
+            }
+            if (j == 0) nck[(bs * NT + n) * A + a] = cj;
+        }
+        if (kq_decay) {   // the Q-layout keys decayed to T - 1, k_t lam^(T-1-t)
+#pragma unroll
+            for (int i = 0; i < kSeg; i += 2) {
+                bf16x2 kb;
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    // past T (k is zero there) the exponent would grow without bound
+                    const float lag = static_cast<float>(max(T - 1 - (t0 + i + e), 0));
+                    kb[e] = static_cast<bf16>(kv[i + e] * __expf(lg * lag));
+                }
+                kpk[i / 2] = __builtin_bit_cast(uint32_t, kb);
+            }
+        }
+        if ((qQ || kQ) && a < AL && on) {
             // Q layout: this thread's positions 16 j .. 16 j + 15 of slot a are two lanes' 16 bytes
             // (qQ is null where no backward follows, as in a prefill)
 #pragma unroll
@@ -308,14 +421,13 @@ __global__ __launch_bounds__(256) void fwd_stats_kernel(RS rs, const float *__re
                 if (kQ) *reinterpret_cast<uint4 *>(kQ + o) = make_uint4(kpk[4 * h], kpk[4 * h + 1], kpk[4 * h + 2], kpk[4 * h + 3]);
             }
         }
-        if (j == 0 && va) nck[(bs * NT + n) * A + a] = carry;
         float nc = carry;
-        for (int m = 0; m < 4; ++m) nc = lam16 * nc + tot[m][s];
+        for (int m = 0; m < 4 * CW; ++m) nc = lam16 * nc + tot[m][s];
         carry = nc;
-        __syncthreads();   // sq, sk complete; tot free for the next chunk
-        if (qR) {
+        __syncthreads();   // sq, sk complete; tot free for the next group
+        if (qR && on) {
             // R layout: the block's 64 positions x 64 slots are 8 tiles; thread -> 2 lanes of one tile
-            const int tl = threadIdx.x / 32, mt = tl / 4, tf4 = tl % 4;
+            const int tl = threadIdx.x % 256 / 32, mt = tl / 4, tf4 = tl % 4;
             if (a0 + 16 * tf4 < AL) {
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
@@ -326,11 +438,11 @@ __global__ __launch_bounds__(256) void fwd_stats_kernel(RS rs, const float *__re
                 }
             }
         }
-        __syncthreads();   // sq, sk read before the next chunk writes them
+        __syncthreads();   // sq, sk read before the next group writes them
     };
-    for (int n = n0; n < n1; n += 2) {
-        chunk(n, 0);
-        if (n + 1 < n1) chunk(n + 1, 1);
+    for (int n = n0; n < n1; n += 2 * CW) {
+        group(n, 0);
+        if (n + CW < n1) group(n + CW, 1);
     }
 }
 
@@ -610,6 +722,15 @@ __global__ __launch_bounds__(256) void stats_reduce_kernel(const float *__restri
 
 // q16n, k16n: natural bf16 copies (both or neither); qR, kR, qQ, kQ: tiled
 // copies AL slots wide (0: AL = A; AL % 32 == 0, the slots past A zero).
+namespace {
+template <class RS, int QW, bool HAS_Q, int CW, class... Args>
+int launch_fwd_stats_cw(dim3 grid, hipStream_t s, Args... args) {
+    constexpr int lds = CW * (2 * ULM_CHUNK * (kSlots + 8) * 2 + 4 * kSlots * 4);
+    fwd_stats_kernel<RS, QW, HAS_Q, CW><<<grid, 256 * CW, lds, s>>>(args...);
+    return check_launch("fwd_stats_kernel");
+}
+}  // namespace
+
 int launch_fwd_stats(const RSrc &src, const float *w, const float *g, float *q, uint16_t *q16n, uint16_t *k16n,
                      uint16_t *qR, uint16_t *kR, uint16_t *qQ, uint16_t *kQ, float *nck, float *c_last, int B, int T,
                      int A, hipStream_t s, void *qw, int qw_dt, int AL, float *segtot, int kq_decay) {
@@ -634,26 +755,32 @@ int launch_fwd_stats(const RSrc &src, const float *w, const float *g, float *q, 
             ULM_TRY(check_launch("fwd_segtot_kernel"));
         }
         const dim3 grid((A + kSlots - 1) / kSlots, B, S);
+        // two chunks side by side where there are fewer workgroups than CUs: 35.6 us against 39.6 at 120 of them
+        // (A = 1912, T = 999), 12.6 against 15.2 at 96 (712, 200), 7.6 against 10.3 at 48 (3072, 117); past that
+        // the larger workgroups leave a shorter last round of CUs: 27.4 against 23.9 at 384 (712, 256). Four side
+        // by side have 128 registers a lane, and spill: 50, 14, 11 and 31.
+        const bool two = NT > 1 && static_cast<size_t>(grid.x) * B * S < 256;
 #define ULM_FWD_STATS(QWK, HQ)                                                                                    \
-    fwd_stats_kernel<RS, QWK, HQ><<<grid, 256, 0, s>>>(rs, w, g, q, qw, qw_dt, q16n, k16n, qR, kR, qQ, kQ, nck,   \
-                                                       c_last, T, A, AL, NT, segtot, S, kq_decay)
+    return two ? launch_fwd_stats_cw<RS, QWK, HQ, 2>(grid, s, rs, w, g, q, qw, qw_dt, q16n, k16n, qR, kR, qQ, \
+                                                         kQ, nck, c_last, T, A, AL, NT, segtot, S, kq_decay)      \
+                   : launch_fwd_stats_cw<RS, QWK, HQ, 1>(grid, s, rs, w, g, q, qw, qw_dt, q16n, k16n, qR, kR, qQ, \
+                                                         kQ, nck, c_last, T, A, AL, NT, segtot, S, kq_decay)
         if (q) {
             switch (qwk) {
-            case ULM_F32: ULM_FWD_STATS(ULM_F32, true); break;
-            case ULM_BF16: ULM_FWD_STATS(ULM_BF16, true); break;
-            case ULM_F16: ULM_FWD_STATS(ULM_F16, true); break;
-            default: ULM_FWD_STATS(-1, true); break;
+            case ULM_F32: ULM_FWD_STATS(ULM_F32, true);
+            case ULM_BF16: ULM_FWD_STATS(ULM_BF16, true);
+            case ULM_F16: ULM_FWD_STATS(ULM_F16, true);
+            default: ULM_FWD_STATS(-1, true);
             }
         } else {
             switch (qwk) {
-            case ULM_F32: ULM_FWD_STATS(ULM_F32, false); break;
-            case ULM_BF16: ULM_FWD_STATS(ULM_BF16, false); break;
-            case ULM_F16: ULM_FWD_STATS(ULM_F16, false); break;
-            default: ULM_FWD_STATS(-1, false); break;
+            case ULM_F32: ULM_FWD_STATS(ULM_F32, false);
+            case ULM_BF16: ULM_FWD_STATS(ULM_BF16, false);
+            case ULM_F16: ULM_FWD_STATS(ULM_F16, false);
+            default: ULM_FWD_STATS(-1, false);
             }
         }
 #undef ULM_FWD_STATS
-        return check_launch("fwd_stats_kernel");
     });
 }
 
