@@ -92,3 +92,18 @@ def test_left_to_the_per_kernel_form():
         before = {k: s[k].clone() for k in ("S", "c", "r_prev", "buf")}
         assert model_mod.decode_step(torch.randn(N, 64, device="cuda"), [s], [1e-5]) is None
         assert s["np"] == 0 and all(torch.equal(s[k], t) for k, t in before.items())
+
+
+def test_final_norm_in_one_launch():
+    """The step's last norm against the module: rsqrt of a D-term mean, a few roundings of 6e-8; a hooked norm
+    goes through its module."""
+    lm = _block(100, 64, 4, 2)
+    say("UnifiedLM.step: the final norm in one launch")
+    with torch.no_grad():
+        lm.norm.weight.normal_()
+        h = torch.randn(5, 100, device="cuda")
+        assert rel(lm._final_norm(h), lm.norm(h)) < 1e-6
+        seen = []
+        lm.norm.register_forward_hook(lambda m, i, o: seen.append(o))
+        lm.step(torch.zeros(2, dtype=torch.long, device="cuda"), lm.init_states(2, "cuda"))
+    assert len(seen) == 1

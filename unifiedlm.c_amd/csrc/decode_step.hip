@@ -7,7 +7,7 @@
 // per-kernel form (RMSNorm + conv, three GEMMs, address, state read: 6 launches
 // and their host work) took 93 us per block and position at 8 sequences of the
 // 110M widths and 99 us per block of the default model at one, against 14 and
-// 1 us of bytes; this form takes 32 and 12 us. What depends on what leaves two
+// 1 us of bytes; this form takes 30 and 11 us. What depends on what leaves two
 // phases with one grid-wide dependency between them, the address's row sum:
 //
 //   in    h, u (RMSNorm, conv) formed by every workgroup for itself;
@@ -43,6 +43,7 @@ constexpr int kLdsFloats = 15 * 1024;   // of dynamic LDS per workgroup: 60 KB
 constexpr int kRows = 4;          // weight rows per wave
 constexpr int kWaves = 8;         // waves per workgroup of the first phase
 constexpr int kTile = kRows * kWaves;   // rows per workgroup: 32, half a wave's lanes in the epilogue
+constexpr int kMaxTaps = 8;
 constexpr int kCus = 256;
 constexpr int kGroup = 4;         // sequences per workgroup of the second phase
 constexpr int kParts = kMaxPending + 2;   // row stride of the partial sums: z, then the pending terms
@@ -305,8 +306,9 @@ __global__ __launch_bounds__(kWaves * 64) void decode_in_kernel(Layer L, const f
 // against q's slice in LDS, KB slices at a time with the next KB in flight. q
 // goes into LDS without the address's 1 / denom, which multiplies the read-out
 // instead: the stream waits for q alone, and wave i sums sequence n0 + i's
-// parts beside it. 20 us at N = 8 and the 110M widths (75 MB of S_base), 6 us at
-// N = 1 and the default model's; a whole row of one sequence after the other,
+// parts beside it. 18 us at N = 8 and the 110M widths (75 MB of S_base), 5.6 us
+// at N = 1 and the default model's (20 and 6.2 with the parts, the address and
+// the windows loaded where they are used); a whole row of one sequence after the other,
 // with its prologue ahead of the stream, took 24. A % 4 == 0, nta <= 128.
 template <int NG>
 __global__ __launch_bounds__(512) void decode_out_kernel(Layer L, const float *__restrict__ x,
@@ -339,40 +341,56 @@ __global__ __launch_bounds__(512) void decode_out_kernel(Layer L, const float *_
             wv[b][u] = *at16(L.w, off);
         }
     };
-    // q: the sequences' rows are one contiguous range
+    // Loads complete in order and the stream waits for q alone, so q is asked for
+    // first; then everything else that is small, so that nothing is asked for at
+    // the end: the parts (wave i: sequence n0 + i's; values past the m + 2 in use
+    // read the row sum's again, unused), this thread's share of the address and of
+    // the conv windows.
     constexpr int QB = 8;
     const f32x4 *zr = reinterpret_cast<const f32x4 *>(zq + static_cast<size_t>(n0) * A);
     const int nq = ng * A4, nt = blockDim.x;
     f32x4 qv[QB];
 #pragma unroll
-    for (int u = 0; u < QB; ++u) qv[u] = zr[min(tid + u * nt, nq - 1)];
+    for (int u = 0; u < QB; ++u) qv[u] = zr[min(tid + u * nt, nq - 1)];   // the sequences' rows are contiguous
+    const float *pn = part + static_cast<size_t>(n0 + min(wave, ng - 1)) * kParts * nta;
+    float v[32], v2[kParts];
+#pragma unroll
+    for (int i = 0; i < kParts; ++i) v[i] = ld_row(pn + (i <= mt ? i : 0) * nta, 4u * min(lane, nta - 1));
+#pragma unroll
+    for (int i = 0; i < kParts; ++i) v2[i] = ld_row(pn + (i <= mt ? i : 0) * nta, 4u * min(lane + 64, nta - 1));
+    const int gi = blockIdx.x * nt + tid;   // 16-byte slice gi of the sequences' addresses
+    const f32x4 zv = reinterpret_cast<const f32x4 *>(z + static_cast<size_t>(n0) * A)[min(gi, nq - 1)];
+    const int kw = Kc - 1, wi = gi;         // pair (sequence, feature) wi of the sequences' windows
+    const bool shifts = kw > 0 && wi < ng * D;
+    float *win = L.buf + (static_cast<size_t>(n0) * D + (shifts ? wi : 0)) * kw;
+    const float hv = h[static_cast<size_t>(n0) * D + (shifts ? wi : 0)];
+    // one tap leaves no window (and a null buffer): h stands in for it, unused
+    const float *win_in = kw > 0 ? win : h;
+    float st[kMaxTaps - 1];
+#pragma unroll
+    for (int j = 1; j < kMaxTaps - 1; ++j) st[j] = win_in[j < kw ? j : 0];
     load(0, 0);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < QB; ++u)
         if (tid + u * nt < nq) reinterpret_cast<f32x4 *>(sq)[tid + u * nt] = qv[u];
     for (int i = tid + QB * nt; i < nq; i += nt) reinterpret_cast<f32x4 *>(sq)[i] = zr[i];
     const float lam = __expf(L.g[0]);
     __syncthreads();
-    // the first phase's parts, summed while the state streams; their loads
-    // unconditional (values past the m + 2 in use read the row sum's parts again)
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
     if (wave < ng) {
-        const float *pn = part + static_cast<size_t>(n0 + wave) * kParts * nta;
-        float v[32];
 #pragma unroll
-        for (int i = 0; i < kParts; ++i) v[i] = ld_row(pn + (i <= mt ? i : 0) * nta, 4u * min(lane, nta - 1));
-        if (nta > 64) {
-            float t[kParts];
-#pragma unroll
-            for (int i = 0; i < kParts; ++i) t[i] = ld_row(pn + (i <= mt ? i : 0) * nta, 4u * min(lane + 64, nta - 1));
-#pragma unroll
-            for (int i = 0; i < kParts; ++i) v[i] += lane + 64 < nta ? t[i] : 0.f;
-        }
-#pragma unroll
-        for (int i = 0; i < 32; ++i) v[i] = i < kParts && lane < nta ? v[i] : 0.f;
+        for (int i = 0; i < 32; ++i)
+            v[i] = i < kParts ? (lane < nta ? v[i] : 0.f) + (lane + 64 < nta ? v2[i < kParts ? i : 0] : 0.f) : 0.f;
         float s = reduce_scatter<32, 32>(v, lane);
         for (int e = lane / 2 - 1; e >= 0 && e < L.m; ++e) s *= lam;   // term j's weight
         if (lane % 2 == 0) sums[wave][lane / 2] = s;
+    }
+    if (shifts) {
+#pragma unroll
+        for (int j = 1; j < kMaxTaps - 1; ++j)
+            if (j < kw) win[j - 1] = st[j];
+        win[kw - 1] = hv;
     }
     // lane j's pending value
     float pvl[NG];
@@ -408,12 +426,12 @@ __global__ __launch_bounds__(512) void decode_out_kernel(Layer L, const float *_
         add(k0 + KB, 1);
     }
     __syncthreads();
-    if (blockIdx.x == 0 && wave < ng) {   // the address itself, read by the next position
-        const float idn = 1.f / (eps + sums[wave][0]);
-        const size_t o = static_cast<size_t>(n0 + wave) * A;
-        for (int j = lane; j < A4; j += 64)
-            reinterpret_cast<f32x4 *>(L.r_prev + o)[j] = reinterpret_cast<const f32x4 *>(z + o)[j] * idn;
-    }
+    // the address itself, read by the next position (the grid has a thread for every slice: four features' waves at
+    // least per workgroup; the loop covers the shapes where it has not)
+    if (gi < nq) reinterpret_cast<f32x4 *>(L.r_prev + static_cast<size_t>(n0) * A)[gi] = zv * (1.f / (eps + sums[gi / A4][0]));
+    for (int i = gi + gridDim.x * nt; i < nq; i += gridDim.x * nt)
+        reinterpret_cast<f32x4 *>(L.r_prev + static_cast<size_t>(n0) * A)[i] =
+            reinterpret_cast<const f32x4 *>(z + static_cast<size_t>(n0) * A)[i] * (1.f / (eps + sums[i / A4][0]));
 #pragma unroll
     for (int n = 0; n < NG; ++n) acc[n] += lane < mt && n < ng ? pvl[n] * sums[n][1 + lane] : 0.f;
     const float y = reduce_scatter<4, 32>(acc, lane);   // lane 16 n: sequence n0 + n
@@ -421,14 +439,6 @@ __global__ __launch_bounds__(512) void decode_out_kernel(Layer L, const float *_
     if (lane % 16 == 0 && n < ng && d < D) {
         const size_t o = static_cast<size_t>(n0 + n) * D + d;
         out[o] = x[o] + y * (1.f / (eps + sums[n][0]));
-    }
-    // the conv windows: thread i of the grid shifts pair (sequence, feature) i
-    const int kw = Kc - 1;
-    const size_t gid = (static_cast<size_t>(blockIdx.y) * gridDim.x + blockIdx.x) * blockDim.x + tid;
-    if (kw > 0 && gid < static_cast<size_t>(N) * D) {
-        float *st = L.buf + gid * kw;
-        for (int j = 0; j + 1 < kw; ++j) st[j] = st[j + 1];
-        st[kw - 1] = h[gid];
     }
 }
 
@@ -504,7 +514,7 @@ using namespace ulm;
 
 // the shapes this form takes; at least one sequence's u fits the LDS of a workgroup
 static bool step_supported(int N, int D, int A, int Kc) {
-    return N >= 1 && N <= step::kMaxN && D >= 1 && A >= 4 && A % 4 == 0 && A <= 4096 && Kc >= 1 && Kc <= 8 &&
+    return N >= 1 && N <= step::kMaxN && D >= 1 && A >= 4 && A % 4 == 0 && A <= 4096 && Kc >= 1 && Kc <= step::kMaxTaps &&
            step::in_groups(N, D) > 0 && 4ull * N * D * A <= step::kMaxState;
 }
 

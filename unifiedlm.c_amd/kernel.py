@@ -680,6 +680,20 @@ def decode_pre(x, norm_w, conv_w, conv_buf, norm_eps):
     return h, u
 
 
+def rms_norm(x, weight, eps):
+    """RMSNorm of a decode position's x (N, D) in one launch (ulm_decode_pre
+    with a conv of one tap, whose output is not used), or None for other
+    dtypes and layouts; no autograd."""
+    if (not _plain_eager(x, weight) or x.dim() != 2 or x.shape[1:] != weight.shape or x.numel() == 0
+            or not (x.is_cuda and x.dtype == weight.dtype == torch.float32 and x.device == weight.device)
+            or not (x.is_contiguous() and weight.is_contiguous())):
+        return None
+    h, u = torch.empty_like(x), torch.empty_like(x)
+    call("ulm_decode_pre", ptr(x), ptr(weight), ptr(weight), None, ptr(h), ptr(u), x.shape[0], x.shape[1], 1, float(eps),
+         nat.stream_of(x))
+    return h
+
+
 def decode_addr(pre, bias, log_eps, w, g, r_prev, c):
     """r = relu^2 address, c <- lam c + (1-lam) w + r_prev (in place), q = r / c.
     Returns (r, q, w*q)."""

@@ -30,7 +30,10 @@ import torch.nn.functional as F
 
 from kernel import (CHUNK, LOG_W_MAX, LOG_W_MIN, block_eager, block_prefill, block_prefill_eager, decode_addr,
                     decode_addr_deferred, decode_deferred, decode_pre, decode_state, decode_step, fm_prefill,
-                    relu2_address, unified_block, unified_memory)
+                    relu2_address, rms_norm, unified_block, unified_memory)
+
+# whether any hook is registered for every module (assumed where torch does not say)
+_any_global_hook = getattr(nn.modules.module, "_has_any_global_hook", lambda: True)
 
 
 @dataclass
@@ -360,11 +363,21 @@ class UnifiedLM(nn.Module):
         """One position for a batch of sequences: tokens (B,) -> logits (B, V)."""
         h = self.tok_embeddings(tokens)
         out = self._few_steps(h, states)
-        if out is None:
-            for layer, s in zip(self.layers, states):
-                h = layer.step(h, s)
-            out = h
-        return self.output(self.norm(out))
+        if out is not None:
+            return self.output(self._final_norm(out))
+        for layer, s in zip(self.layers, states):
+            h = layer.step(h, s)
+        return self.output(self.norm(h))
+
+    def _final_norm(self, h):
+        """self.norm(h) in one launch, unless the module is another one or is hooked."""
+        norm = self.norm
+        if (type(norm) is RMSNorm and "forward" not in norm.__dict__
+                and not (norm._forward_hooks or norm._forward_pre_hooks or _any_global_hook())):
+            out = rms_norm(h, norm.weight, norm.eps)
+            if out is not None:
+                return out
+        return norm(h)
 
     def _few_steps(self, h, states):
         """Every block's step in one native call (kernel.decode_step), or None
