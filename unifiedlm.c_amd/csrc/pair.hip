@@ -99,7 +99,7 @@ enum Epi { EPI_SCORES = 0, EPI_DSCORES = 1, EPI_ROWS = 2, EPI_DQSTATS = 3 };
 // plus an fp32 residual, OUT_DRADD the backward's dr accumulation of dk_f
 constexpr int OUT_DRADD = 6;
 enum KRange { K_FULL = 0, K_CAUSAL = 1, K_ANTI = 2 };
-// EPI_SCORES with fewer 128 x 128 tile jobs than CUs: one workgroup per CU
+// EPI_SCORES with fewer 128 x 128 tile jobs than CUs (and more than few_tiles): one workgroup per CU
 // holds them all, so its stages go to depth instead (96 KB: five k-steps of
 // copies in flight instead of two, against the latency of each k-step's reads)
 constexpr int kScoresDeep = 1;
@@ -199,6 +199,21 @@ __device__ __forceinline__ void wait_copies(int ksteps) {
     default: __builtin_amdgcn_s_waitcnt(waitcnt_vm(4 * LPW)); break;
     }
 }
+
+// Whether pair_small_kernel takes the scores and dscores, by their number of
+// 128 x 128 tiles (its waves are 16 times as many). us, pair_kernel against it:
+//   tiles, 32-element steps    scores          steps   dscores
+//   1 (3072 slots)     96      31.0 / 10.5
+//   16                 64      24.5 / 10.4     16      13.7 / 8.5
+//   24                 23      14.7 /  7.8      9      12.8 / 8.3
+//   36                 96      32.3 / 15.9     24      14.9 / 10.0
+//   48                 23      15.4 / 10.1      9      12.1 / 9.7
+//   72                 64      25.0 / 25.5     16      12.9 / 11.9
+//   80                  4       9.5 / 12.1      2       9.6 / 9.0
+//   96                 23      15.8 / 18.1      9      13.5 / 12.0
+//   144                60      26.1 / 37.5     24      18.1 / 22.8
+inline bool few_tiles(int tiles) { return tiles <= 64; }
+constexpr int kSmallSub = 16;   // its 32 x 32 tiles in a 128 x 128 one
 
 // Output element types of the row epilogue: OUT % 3 = ulm_dtype of the
 // output, OUT >= 3 adds an fp32 residual; the statistics epilogue uses OUT
@@ -963,6 +978,156 @@ __global__ __launch_bounds__((waves_of<TM, EPI>() * 64), (min_blocks<TM, EPI, OU
     }
 }
 
+// The scores and dscores where their 128 x 128 tiles are few: one wave per
+// 32 x 32 tile. At such a shape a 128 x 128 tile's k-loop is a chain of copies
+// into LDS and barriers, about 0.3 us a 32-element step, on a few CUs: 30 us for
+// one 117-position prompt's 96 steps. Here a wave reads its MFMA operands from
+// the tiled copies straight into registers (a tile is one operand, 1 KB, in one
+// load), U steps at a time with the next U in flight and no barrier, in the
+// same order of steps as pair_kernel, so that a row's scores have the same bits
+// whatever the batch (the contraction split over a workgroup's waves, their sums
+// joined through LDS, took as long and lost that). The epilogue's items are 8
+// consecutive s of one t (P or dS and P's residual, 16 bytes each) and then 8
+// consecutive t of one s (the transposes). Tiles above the diagonal of a
+// 128 x 128 block are zeros (the products read whole blocks). A workgroup is
+// four waves for the sake of the tile copies that ride along; a tile's uses one.
+// Timed below, at few_tiles.
+template <int EPI>
+__global__ __launch_bounds__(256) void pair_small_kernel(Args p) {
+    constexpr int TS = 32, SUB = 128 / TS, XS = TS + 1;
+    constexpr int U = 8;
+    extern __shared__ __align__(16) char lds[];
+    if constexpr (EPI == EPI_SCORES) {
+        // the v tile copies, as in pair_kernel
+        if (static_cast<int>(blockIdx.x) >= p.jobs) {
+            const int job = static_cast<int>(blockIdx.x) - p.jobs;
+            const int per_b = p.cp_gx * p.NT;
+            tile_copy_bf16(p.cp_src, p.cp_q, p.cp_r, p.T, p.cp_X, p.NT, (job % p.cp_gx) * kCopyBlocks * ULM_CHUNK,
+                           (job % per_b) / p.cp_gx, job / per_b, threadIdx.x, true, reinterpret_cast<copy_tile_t *>(lds));
+            return;
+        }
+    }
+    if (threadIdx.x >= 64) return;
+    float *X = reinterpret_cast<float *>(lds);   // [TS s][XS]
+    const int lane = threadIdx.x;
+    int logical = blockIdx.x;
+    if (p.jobs % 8 == 0) logical = (blockIdx.x % 8) * (p.jobs / 8) + blockIdx.x / 8;   // XCD-local rows
+    const int b = logical / p.jobs_per_row, job = logical % p.jobs_per_row;
+    int mb, nb;
+    job_tiles(p, job / (SUB * SUB), mb, nb);
+    const int s0 = mb * 128 + (job % SUB) * TS, t0 = nb * 128 + (job / SUB) % SUB * TS;
+    const bool dots = s0 < t0 + TS && t0 < p.T;
+    if (dots) {
+        f32x16 acc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+        const rsrc_t ra = rsrc(reinterpret_cast<const char *>(p.a.p) + b * p.a.bstride, p.a.bstride);
+        const rsrc_t rb = rsrc(reinterpret_cast<const char *>(p.b.p) + b * p.b.bstride, p.b.bstride);
+        // row tiles (past the rows: past the range)
+        const uint32_t oa = (s0 / 32 * p.a.rt + 16u * lane) | (s0 / 32 < p.a.nrt ? 0u : OOB);
+        const uint32_t ob = (t0 / 32 * p.b.rt + 16u * lane) | (t0 / 32 < p.b.nrt ? 0u : OOB);
+        bf16x8 fa[2][U], fb[2][U];
+        const int nk = p.a.nkt;
+        auto load = [&](int k0, int st) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int k = k0 + u;
+                const uint32_t off = (k / 4) * p.a.ks + (k % 4) * TB, past = k < nk ? 0u : OOB;   // both R layout: the same steps
+                fa[st][u] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(ra, (oa + off) | past, 0, 0));
+                fb[st][u] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(rb, (ob + off) | past, 0, 0));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto add = [&](int st) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) acc = mfma(fa[st][u], fb[st][u], acc);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        load(0, 0);
+        for (int k = 0; k < nk; k += 2 * U) {   // steps past the contraction read zeros, without traffic
+            load(k + U, 1);
+            add(0);
+            load(k + 2 * U, 0);
+            add(1);
+        }
+        const int h = lane / 32, lc = lane % 32;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float x = acc[r];
+            X[(8 * (r / 4) + 4 * h + r % 4) * XS + lc] = x;
+        }
+        __builtin_amdgcn_s_waitcnt(kWaitLgkm0);   // the tile's one wave: its writes before its reads
+        __builtin_amdgcn_wave_barrier();
+    }
+    const float g = p.g[0];
+    const bool want_t = p.pout_t != nullptr;
+    const rsrc_t rp = rsrc(reinterpret_cast<char *>(p.pout) + b * p.p_bstride, p.p_bstride);
+    const rsrc_t rpt = rsrc(want_t ? reinterpret_cast<char *>(p.pout_t) + b * p.p_bstride : nullptr, want_t ? p.p_bstride : 0);
+    const rsrc_t rpin = rsrc(EPI == EPI_DSCORES ? reinterpret_cast<const char *>(p.pin) + b * p.p_bstride
+                                                : reinterpret_cast<const char *>(p.pout), p.p_bstride);
+    const char *lo = EPI == EPI_DSCORES ? reinterpret_cast<const char *>(p.pin_lo) : reinterpret_cast<const char *>(p.pout_lo);
+    const rsrc_t rplo = rsrc(lo ? lo + b * p.p_bstride : nullptr, lo ? p.p_bstride : 0);
+    auto value = [&](int s, int t) {   // the decayed, masked element (s, t) of the tile
+        const bool ok = dots && s0 + s <= t0 + t && t0 + t < p.T;
+        return ok ? X[s * XS + t] * __expf(g * static_cast<float>(t0 + t - s0 - s)) : 0.f;
+    };
+    // P-layout byte of (row r, contraction c), c a multiple of 8
+    auto at = [&](int r, int c) -> uint32_t { return (r / 32) * p.p_rt + (c / 16) * TB + 16u * (r % 32 + 32 * ((c % 16) / 8)); };
+    constexpr int T8 = TS * TS / 8;
+    float dg = 0.f;
+    for (int e = lane; e < T8; e += 64) {
+        const int t = e % TS, s8 = 8 * (e / TS);
+        const uint32_t off = at(t0 + t, s0 + s8);
+        v4f32_t pv, pl;
+        if constexpr (EPI == EPI_DSCORES) {
+            pv = __builtin_bit_cast(v4f32_t, __builtin_amdgcn_raw_buffer_load_b128(rpin, off, 0, 0));
+            pl = __builtin_bit_cast(v4f32_t, __builtin_amdgcn_raw_buffer_load_b128(rplo, off, 0, 0));
+        }
+        uint32_t hi[4], rem[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            float x[2];
+            uint16_t xb[2], lb[2];
+#pragma unroll
+            for (int e2 = 0; e2 < 2; ++e2) {
+                const int s = s8 + 2 * k + e2;
+                x[e2] = value(s, t);
+                xb[e2] = f32_to_bf16_bits(x[e2]);
+                lb[e2] = f32_to_bf16_bits(x[e2] - bf16_to_f32(xb[e2]));
+                if constexpr (EPI == EPI_DSCORES) {
+                    // P to about 16 significant bits (see pair_kernel's epilogue)
+                    const float pe = bf16_to_f32((__float_as_uint(pv[k]) >> (16 * e2)) & 0xffffu) +
+                                     bf16_to_f32((__float_as_uint(pl[k]) >> (16 * e2)) & 0xffffu);
+                    if (dots && s0 + s <= t0 + t && t0 + t < p.T)
+                        dg += static_cast<float>(t0 + t - s0 - s) * pe * X[s * XS + t];
+                }
+            }
+            hi[k] = static_cast<uint32_t>(xb[0]) | (static_cast<uint32_t>(xb[1]) << 16);
+            rem[k] = static_cast<uint32_t>(lb[0]) | (static_cast<uint32_t>(lb[1]) << 16);
+        }
+        const gv4u32_t v = {hi[0], hi[1], hi[2], hi[3]};
+        __builtin_amdgcn_raw_buffer_store_b128(v, rp, off, 0, 0);
+        if constexpr (EPI == EPI_SCORES) {
+            const gv4u32_t vl = {rem[0], rem[1], rem[2], rem[3]};
+            __builtin_amdgcn_raw_buffer_store_b128(vl, rplo, off, 0, 0);
+        }
+    }
+    for (int e = lane; want_t && e < T8; e += 64) {
+        const int s = e % TS, t8 = 8 * (e / TS);
+        uint32_t hi[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            hi[k] = static_cast<uint32_t>(f32_to_bf16_bits(value(s, t8 + 2 * k))) |
+                    (static_cast<uint32_t>(f32_to_bf16_bits(value(s, t8 + 2 * k + 1))) << 16);
+        const gv4u32_t v = {hi[0], hi[1], hi[2], hi[3]};
+        __builtin_amdgcn_raw_buffer_store_b128(v, rpt, at(s0 + s, t0 + t8), 0, 0);
+    }
+    if constexpr (EPI == EPI_DSCORES) {
+        const double w = wave_sum(static_cast<double>(dg));
+        if (lane == 0) p.dg_part[logical] = w;
+    }
+}
+
 // dw[a] = sum over batch rows of sum over tiles (last first) of the tiles'
 // dw parts, in that fixed order: blocks of 16 slots x 16 batch rows, the rows
 // summed through LDS. The last block sums the n1 + n2 decay-gradient partials
@@ -1076,6 +1241,21 @@ int launch_g(Args a, int B, hipStream_t s) {
     return la_timer_end(s);
 }
 
+// pair_small_kernel over the 128 x 128 blocks of a.mt tiles a side, tri (job_tiles): 16 jobs each
+template <int EPI>
+int launch_small(Args a, int B, hipStream_t s) {
+    constexpr int lds = EPI == EPI_SCORES ? static_cast<int>(kCopyLds) : 32 * 33 * 4;
+    a.jobs_per_row = a.mt * (a.mt + 1) / 2 * kSmallSub;
+    a.jobs = B * a.jobs_per_row;
+    const int grid = a.jobs + (EPI == EPI_SCORES ? a.cp_jobs : 0);
+    int st = la_timer_begin(s, a.tag);
+    if (st) return st;
+    pair_small_kernel<EPI><<<dim3(static_cast<unsigned>(grid)), 256, lds, s>>>(a);
+    st = check_launch("pair_small_kernel");
+    if (st) return st;
+    return la_timer_end(s);
+}
+
 template <bool TA, bool TBt, int EPI, int OUT>
 int launch_o(const Args &a, int G, int B, hipStream_t s) {
     if constexpr (EPI == EPI_SCORES) {
@@ -1103,9 +1283,11 @@ int launch(const Args &a, int G, int B, hipStream_t s) {
         }
     } else if constexpr (EPI == EPI_SCORES) {
         const int tiles = B * (a.tri ? a.mt * (a.mt + 1) / 2 : a.mt * a.nt);
+        if (G == 128 && few_tiles(tiles)) return launch_small<EPI>(a, B, s);
         if (G == 128 && tiles < 256) return launch_g<128, TA, false, EPI, kScoresDeep>(a, B, s);
         return launch_o<TA, false, EPI, 0>(a, G, B, s);
-    } else if constexpr (EPI != EPI_ROWS) {
+    } else if constexpr (EPI == EPI_DSCORES) {
+        if (few_tiles(B * a.mt * (a.mt + 1) / 2)) return launch_small<EPI>(a, B, s);
         return launch_o<TA, false, EPI, 0>(a, G, B, s);
     } else {
         if (a.drtile) return launch_o<TA, false, EPI, OUT_DRADD>(a, G, B, s);
@@ -1139,8 +1321,8 @@ size_t pair_p_bytes(int B, int T) {
     return static_cast<size_t>(B) * Tq * Tq * 2;
 }
 int pair_dscore_jobs(int B, int T) {
-    const int nb = pair_tq(B, T) / pair_block(B, T);
-    return B * nb * (nb + 1) / 2;
+    const int nb = pair_tq(B, T) / pair_block(B, T), tiles = B * nb * (nb + 1) / 2;
+    return pair::few_tiles(tiles) ? tiles * pair::kSmallSub : tiles;
 }
 
 // Flops per token of the six block-pair products, fwd + bwd, with their
