@@ -16,7 +16,7 @@ from kernel import fm_prefill, unified_memory  # noqa: E402
 
 @pytest.mark.parametrize("T,A,D,dtype", [(1, 32, 32, "bf16"), (31, 40, 33, "fp32"), (33, 300, 64, "bf16"),
                                          (100, 71, 288, "bf16"), (128, 128, 96, "bf16"), (130, 96, 40, "fp32"),
-                                         (300, 64, 32, "bf16")])
+                                         (300, 64, 32, "bf16"), (129, 64, 96, "fp16")])
 def test_rows_alone_and_among_many(T, A, D, dtype, monkeypatch):
     monkeypatch.setenv("ULM_FM_PATH", "pair")
     tiles = (T + 127) // 128
@@ -25,7 +25,7 @@ def test_rows_alone_and_among_many(T, A, D, dtype, monkeypatch):
     say(f"few score tiles: rows alone and among {B}, T={T} A={A} D={D} {dtype}")
     gen = torch.Generator(device="cuda").manual_seed(T + A)
     rn = lambda *s: torch.randn(*s, device="cuda", generator=gen)  # noqa: E731
-    dt = torch.bfloat16 if dtype == "bf16" else torch.float32
+    dt = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}[dtype]
     r = rn(B, T, A).clamp(min=0) ** 2 / A
     v, df, dq = rn(B, T, D).to(dt), rn(B, T, D).to(dt), 0.1 * rn(B, T, A)
     g, w = torch.tensor(-0.03, device="cuda"), 4 * torch.exp(0.3 * rn(A))

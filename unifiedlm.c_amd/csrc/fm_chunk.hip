@@ -354,6 +354,9 @@ int la_timer_end(hipStream_t s) {
     return ULM_OK;
 }
 
+// Whether launches are being timed (a launch that holds two products then makes one for each).
+bool la_timer_on() { return g_la_timer.on; }
+
 int launch_partial_reduce(const float *part, int nK, size_t n, void *out, int odt, hipStream_t s,
                           const float *resid);
 

@@ -57,6 +57,7 @@ namespace ulm {
 
 int la_timer_begin(hipStream_t s, int tag);
 int la_timer_end(hipStream_t s);
+bool la_timer_on();
 
 namespace pair {
 
@@ -219,7 +220,7 @@ constexpr int kSmallSub = 16;   // its 32 x 32 tiles in a 128 x 128 one
 // output, OUT >= 3 adds an fp32 residual; the statistics epilogue uses OUT
 // for its input kinds.
 template <int TM, int TN, int KT, bool TA, bool TBt, int EPI, int OUT>
-__global__ __launch_bounds__((waves_of<TM, EPI>() * 64), (min_blocks<TM, EPI, OUT>())) void pair_kernel(Args p) {
+__device__ __forceinline__ void pair_body(const Args &p, const int bid) {
     constexpr int WV = waves_of<TM, EPI>(), WM = WV / 2;   // waves, and waves along m
     constexpr int MI = TM / (32 * WM), NI = TN / 64;       // 32-row / 32-column tiles per wave
     constexpr int KS = 16 * KT;                        // contraction elements per k-step
@@ -236,10 +237,10 @@ __global__ __launch_bounds__((waves_of<TM, EPI>() * 64), (min_blocks<TM, EPI, OU
         // the tile copies ride on the workgroups past the tile jobs: the
         // scores' tiles leave CUs idle, and copies need no MFMA. Each group of
         // 4 waves takes one job with its own part of the stage memory.
-        if (static_cast<int>(blockIdx.x) >= p.jobs) {
+        if (bid >= p.jobs) {
             constexpr int WV = waves_of<TM, EPI>();
             const int grp = threadIdx.x / 256;
-            const int job = (static_cast<int>(blockIdx.x) - p.jobs) * (WV / 4) + grp;
+            const int job = (bid - p.jobs) * (WV / 4) + grp;
             const int per_b = p.cp_gx * p.NT;
             const bool live = job < p.cp_jobs;
             const int jj = live ? job : 0;
@@ -254,8 +255,8 @@ __global__ __launch_bounds__((waves_of<TM, EPI>() * 64), (min_blocks<TM, EPI, OU
     const int lane = threadIdx.x % 64;
     const int wm = wave / 2, wn = wave % 2;
 
-    int logical = blockIdx.x;
-    if (p.jobs % 8 == 0) logical = (blockIdx.x % 8) * (p.jobs / 8) + blockIdx.x / 8;   // XCD-local rows
+    int logical = bid;
+    if (p.jobs % 8 == 0) logical = (bid % 8) * (p.jobs / 8) + bid / 8;   // XCD-local rows
     const int b = logical / p.jobs_per_row;
     int mb, nb;
     job_tiles(p, logical % p.jobs_per_row, mb, nb);
@@ -978,6 +979,11 @@ __global__ __launch_bounds__((waves_of<TM, EPI>() * 64), (min_blocks<TM, EPI, OU
     }
 }
 
+template <int TM, int TN, int KT, bool TA, bool TBt, int EPI, int OUT>
+__global__ __launch_bounds__((waves_of<TM, EPI>() * 64), (min_blocks<TM, EPI, OUT>())) void pair_kernel(Args p) {
+    pair_body<TM, TN, KT, TA, TBt, EPI, OUT>(p, blockIdx.x);
+}
+
 // The scores and dscores where their 128 x 128 tiles are few: one wave per
 // 32 x 32 tile. At such a shape a 128 x 128 tile's k-loop is a chain of copies
 // into LDS and barriers, about 0.3 us a 32-element step, on a few CUs: 30 us for
@@ -993,14 +999,14 @@ __global__ __launch_bounds__((waves_of<TM, EPI>() * 64), (min_blocks<TM, EPI, OU
 // four waves for the sake of the tile copies that ride along; a tile's uses one.
 // Timed below, at few_tiles.
 template <int EPI>
-__global__ __launch_bounds__(256) void pair_small_kernel(Args p) {
+__device__ __forceinline__ void pair_small_body(const Args &p, const int bid) {
     constexpr int TS = 32, SUB = 128 / TS, XS = TS + 1;
     constexpr int U = 8;
     extern __shared__ __align__(16) char lds[];
     if constexpr (EPI == EPI_SCORES) {
         // the v tile copies, as in pair_kernel
-        if (static_cast<int>(blockIdx.x) >= p.jobs) {
-            const int job = static_cast<int>(blockIdx.x) - p.jobs;
+        if (bid >= p.jobs) {
+            const int job = bid - p.jobs;
             const int per_b = p.cp_gx * p.NT;
             tile_copy_bf16(p.cp_src, p.cp_q, p.cp_r, p.T, p.cp_X, p.NT, (job % p.cp_gx) * kCopyBlocks * ULM_CHUNK,
                            (job % per_b) / p.cp_gx, job / per_b, threadIdx.x, true, reinterpret_cast<copy_tile_t *>(lds));
@@ -1010,8 +1016,8 @@ __global__ __launch_bounds__(256) void pair_small_kernel(Args p) {
     if (threadIdx.x >= 64) return;
     float *X = reinterpret_cast<float *>(lds);   // [TS s][XS]
     const int lane = threadIdx.x;
-    int logical = blockIdx.x;
-    if (p.jobs % 8 == 0) logical = (blockIdx.x % 8) * (p.jobs / 8) + blockIdx.x / 8;   // XCD-local rows
+    int logical = bid;
+    if (p.jobs % 8 == 0) logical = (bid % 8) * (p.jobs / 8) + bid / 8;   // XCD-local rows
     const int b = logical / p.jobs_per_row, job = logical % p.jobs_per_row;
     int mb, nb;
     job_tiles(p, job / (SUB * SUB), mb, nb);
@@ -1125,6 +1131,23 @@ __global__ __launch_bounds__(256) void pair_small_kernel(Args p) {
     if constexpr (EPI == EPI_DSCORES) {
         const double w = wave_sum(static_cast<double>(dg));
         if (lane == 0) p.dg_part[logical] = w;
+    }
+}
+
+template <int EPI>
+__global__ __launch_bounds__(256) void pair_small_kernel(Args p) {
+    pair_small_body<EPI>(p, blockIdx.x);
+}
+
+// dscores and dv in one launch, dscores' jobs first: neither needs the other.
+template <bool FEW, int DV_OUT>
+__global__ __launch_bounds__(256, 2) void pair_dual_kernel(Args ds, Args dv) {
+    const int bid = blockIdx.x;
+    if (bid < ds.jobs) {
+        if constexpr (FEW) pair_small_body<EPI_DSCORES>(ds, bid);
+        else pair_body<128, 128, 2, false, false, EPI_DSCORES, 0>(ds, bid);
+    } else {
+        pair_body<128, 128, 2, false, false, EPI_ROWS, DV_OUT>(dv, bid - ds.jobs);
     }
 }
 
@@ -1254,6 +1277,35 @@ int launch_small(Args a, int B, hipStream_t s) {
     st = check_launch("pair_small_kernel");
     if (st) return st;
     return la_timer_end(s);
+}
+
+template <bool FEW, int DV_OUT>
+int launch_dual_as(const Args &ds, const Args &dv, hipStream_t s) {
+    constexpr int lds = nstage<128, EPI_ROWS, DV_OUT>() * 8 * 2 * static_cast<int>(TB);   // the deeper of the two
+    static bool attr_done[64] = {};
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return check_launch("hipGetDevice");
+    if (!attr_done[dev]) {
+        if (hipFuncSetAttribute(reinterpret_cast<const void *>(&pair_dual_kernel<FEW, DV_OUT>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+            return check_launch("pair_dual_kernel attribute");
+        attr_done[dev] = true;
+    }
+    pair_dual_kernel<FEW, DV_OUT><<<dim3(static_cast<unsigned>(ds.jobs + dv.jobs)), 256, lds, s>>>(ds, dv);
+    return check_launch("pair_dual_kernel");
+}
+
+int launch_dual(Args ds, Args dv, int B, hipStream_t s) {
+    const bool few = few_tiles(B * ds.mt * (ds.mt + 1) / 2);
+    ds.jobs_per_row = ds.mt * (ds.mt + 1) / 2 * (few ? kSmallSub : 1);
+    ds.jobs = B * ds.jobs_per_row;
+    dv.jobs_per_row = dv.mt * dv.nt;
+    dv.jobs = B * dv.jobs_per_row;
+    switch (dv.out_dt) {
+    case ULM_F32: return few ? launch_dual_as<true, ULM_F32>(ds, dv, s) : launch_dual_as<false, ULM_F32>(ds, dv, s);
+    case ULM_BF16: return few ? launch_dual_as<true, ULM_BF16>(ds, dv, s) : launch_dual_as<false, ULM_BF16>(ds, dv, s);
+    default: return few ? launch_dual_as<true, ULM_F16>(ds, dv, s) : launch_dual_as<false, ULM_F16>(ds, dv, s);
+    }
 }
 
 template <bool TA, bool TBt, int EPI, int OUT>
@@ -1483,7 +1535,7 @@ namespace {
 // The launches of launch_pair_backward after the fork: dv on the second stream
 // (sd, or s when null), then dscores, dq_f with the statistics, dk_f into dr and
 // the final sums on s.
-int pair_backward_products(const SideStream *sd, const uint16_t *vR, const uint16_t *doR, const uint16_t *doQ,
+int pair_backward_products(const SideStream *sd, bool dual, const uint16_t *vR, const uint16_t *doR, const uint16_t *doQ,
                            const uint16_t *kQ, const uint16_t *qQ, const uint16_t *P, const uint16_t *Pt,
                            const uint16_t *Plo, const float *g, uint16_t *dS, uint16_t *dSt, double *dg_part,
                            const RSrc &rsrc_in, const void *xq, int xq_kind, const float *nck, const float *w,
@@ -1493,8 +1545,8 @@ int pair_backward_products(const SideStream *sd, const uint16_t *vR, const uint1
     const int G = pair_block(B, T), Tq = pair_tq(B, T), NT = (T + 63) / 64, MT = Tq / G;
     const int Ap = (A + 31) / 32 * 32, Dp = (D + 31) / 32 * 32;   // operand tile widths
     const Mat sm = p_mat(dS, Tq);
+    Args d{};
     {
-        Args d{};
         d.T = T;
         d.g = g;
         d.mt = MT;
@@ -1508,7 +1560,7 @@ int pair_backward_products(const SideStream *sd, const uint16_t *vR, const uint1
         d.out_dt = dv_dt;
         d.F = D;
         d.tag = ULM_PRODUCT_DV;
-        ULM_TRY((launch<false, EPI_ROWS>(d, G, B, sd ? sd->s : s)));
+        if (!dual) ULM_TRY((launch<false, EPI_ROWS>(d, G, B, sd ? sd->s : s)));
     }
     Args a{};
     a.T = T;
@@ -1527,7 +1579,8 @@ int pair_backward_products(const SideStream *sd, const uint16_t *vR, const uint1
     a.pin_lo = Plo;
     a.dg_part = dg_part;
     a.tag = ULM_PRODUCT_DSCORES;
-    ULM_TRY((launch<false, EPI_DSCORES>(a, G, B, s)));
+    if (dual) ULM_TRY(launch_dual(a, d, B, s));
+    else ULM_TRY((launch<false, EPI_DSCORES>(a, G, B, s)));
     Args r{};
     r.T = T;
     r.g = g;
@@ -1576,9 +1629,9 @@ int pair_backward_products(const SideStream *sd, const uint16_t *vR, const uint1
 }
 }  // namespace
 
-// The backward: dv = P^T dfast in dv_dt (B, T, D), on the device's second
-// stream (forked from s and joined back into s before the return, so that work
-// later on s is ordered after it); dS = dscores(dfast, v) and its transpose dSt
+// The backward: dv = P^T dfast in dv_dt (B, T, D), in the dscores launch or on
+// the device's second stream (forked from s and joined back into s before the
+// return, so that work later on s is ordered after it); dS = dscores(dfast, v) and its transpose dSt
 // with the pair part of the decay gradient; dq_f = dS k with the per-slot
 // statistics in its epilogue (dr without dk_f and the carry; the tile
 // statistics); dk_f = dS^T q added into dr with the carry of dkc between
@@ -1603,7 +1656,16 @@ int launch_pair_backward(const uint16_t *vR, const uint16_t *doR, const uint16_t
     static std::mutex side_mu;
     const std::lock_guard<std::mutex> lock(side_mu);
     SideStream *sd = nullptr;
-    if (static_cast<double>(B) * Tq * Tq * D >= 2e9) {
+    // ... and where neither fills the device by itself, in the dscores launch
+    // instead: one launch less, no fork. One block fwd + bwd, us, as before / in
+    // one launch, at (dscores + dv) jobs of 128 x 128 tiles: B=32 T=256 D=288
+    // (288) 121 / 116; B=2 T=1024 D=768 (168) 162 / 151; B=4 T=999 D=768 (336,
+    // forked before) 180 / 173; B=8 T=1024 D=512 (544, forked) 200 / 194; but
+    // B=16 T=1024 D=288 (960, forked) 252 / 255, D=768 (1344, forked) 640 / 652.
+    const double work = static_cast<double>(B) * Tq * Tq * D;
+    const int jobs = B * MT * (MT + 1) / 2 + B * MT * ((D + 127) / 128);
+    const bool dual = (work < 2e9 || jobs <= 640) && !la_timer_on();
+    if (!dual && work >= 2e9) {
         ULM_TRY(side_stream(sd));
         if (hipEventRecord(sd->fork, s) != hipSuccess || hipStreamWaitEvent(sd->s, sd->fork, 0) != hipSuccess)
             return check_launch("side stream fork");
@@ -1611,7 +1673,7 @@ int launch_pair_backward(const uint16_t *vR, const uint16_t *doR, const uint16_t
     // From the fork on, every return joins the second stream back into s, the
     // error returns included: the caller frees the workspace (and may reuse dv)
     // in stream order on s once this returns, so s must not run ahead of dv.
-    const int rc = pair_backward_products(sd, vR, doR, doQ, kQ, qQ, P, Pt, Plo, g, dS, dSt, dg_part, rsrc_in, xq,
+    const int rc = pair_backward_products(sd, dual, vR, doR, doQ, kQ, qQ, P, Pt, Plo, g, dS, dSt, dg_part, rsrc_in, xq,
                                           xq_kind, nck, w, dr, dw, dg, st, dv, dv_dt, B, T, A, D, s);
     if (sd && (hipEventRecord(sd->join, sd->s) != hipSuccess || hipStreamWaitEvent(s, sd->join, 0) != hipSuccess)) {
         const int jrc = check_launch("side stream join");
