@@ -55,39 +55,6 @@ struct Layer {
     int m;   // terms already pending: this position's is term m
 };
 
-// Sums v[0 .. V-1] over the 2 * MASK lanes of this lane's group (MASK = 32: the
-// wave, 16: half a wave); lane l of the group ends with the sum of value
-// l / (2 MASK / V): at each step a lane keeps half of its values and hands the
-// other half to the lane across, V - 1 exchanges instead of V log2.
-// Recursive, so that every index into v is a constant: with a loop over the
-// halvings the compiler kept v in select chains thousands of instructions long.
-template <int V, int MASK> __device__ __forceinline__ float reduce_scatter(float (&v)[V], int lane) {
-    if constexpr (V > 1) {
-        const bool up = lane & MASK;
-        float t[V / 2];
-#pragma unroll
-        for (int k = 0; k < V / 2; ++k) {
-            if constexpr (MASK >= 16) {
-                // one instruction exchanges the upper half (or the odd rows of 16) of the one with the lower half
-                // (the even rows) of the other: what this lane keeps and what it is handed, in either order
-                const uint32_t x = __float_as_uint(v[k]), y = __float_as_uint(v[k + V / 2]);
-                const auto r = MASK == 32 ? __builtin_amdgcn_permlane32_swap(x, y, false, false)
-                                          : __builtin_amdgcn_permlane16_swap(x, y, false, false);
-                t[k] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-            } else {
-                const float keep = up ? v[k + V / 2] : v[k], send = up ? v[k] : v[k + V / 2];
-                t[k] = keep + __shfl_xor(send, MASK, kWave);
-            }
-        }
-        return reduce_scatter<V / 2, MASK / 2>(t, lane);
-    } else if constexpr (MASK >= 1) {
-        float t[1] = {v[0] + __shfl_xor(v[0], MASK, kWave)};
-        return reduce_scatter<1, MASK / 2>(t, lane);
-    } else {
-        return v[0];
-    }
-}
-
 // V consecutive floats at p, in one access where V is 4 (16-byte aligned)
 template <int V> struct Vec {
     float e[V];
