@@ -137,21 +137,7 @@ Path train_path(int B, int T, int A, int D) {
     if (env && env[0] == 'c') return PATH_CHUNKED;
     if (!pair_ok) return PATH_CHUNKED;
     if (env && env[0] == 'p') return PATH_PAIR;
-    if (pair < 0.8 * chunked) return PATH_PAIR;
-    // The state form walks the chunks of a row one after the other, on
-    // B ceil(A / 64) workgroups in its widest products: where those leave CUs
-    // idle, or pay each chunk's latency for little work, its flops take longer
-    // than the pair products' do. Flops for which both forms took the same time,
-    // pair over state, by the workgroups w: about 12 at 8, 5.7 at 64, 3.2 at 128,
-    // 2.1 at 256, 1.5 past that (fwd + bwd of one block, the widths of the 260K,
-    // 42M and 110M shapes and between, 512 to 4096 positions: 187 against 109 us
-    // at B = 8, T = 512, A = 128, D = 64; 575 against 203 at 2, 2048, 512, 256;
-    // 532 against 621 at 128, 1024, 128, 64). One tile of positions (T <= 128)
-    // leaves the pair form nothing to spread, and past 2048 positions its saved
-    // scores, 6 Tq^2 bytes a row, are the larger part of a step's memory.
-    const double w = std::min(300.0, static_cast<double>(B) * ((A + 63) / 64));
-    const double scores = 3.0 * static_cast<double>(pair_p_bytes(B, T));
-    return T > 128 && T <= 2048 && scores <= 512e6 && pair * (0.06 + 0.002 * w) < chunked ? PATH_PAIR : PATH_CHUNKED;
+    return pair < 0.8 * chunked ? PATH_PAIR : PATH_CHUNKED;
 }
 
 // The form of a prefill, a forward that also emits the decode state after
