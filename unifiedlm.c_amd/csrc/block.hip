@@ -286,7 +286,7 @@ __global__ __launch_bounds__(kColsMaxD) void norm_conv_bwd_cols_kernel(
 #pragma unroll
     for (int m = 0; m < kMaxTaps; ++m) ca[m] = m < Kc ? ca[m] : 0.f;
     const float nwd = vd ? nw0 : 0.f;
-    float g2[kMaxTaps], dh[kColTP], rd[kColTP];
+    float g2[kMaxTaps], dh[kColTP], an[kColTP];
 #pragma unroll
     for (int m = 0; m < kMaxTaps; ++m) g2[m] = 0.f;
     float gnw = 0.f;
@@ -303,9 +303,9 @@ __global__ __launch_bounds__(kColsMaxD) void norm_conv_bwd_cols_kernel(
         dh[i] = a;
         gnw += a * xn;
         xv[i] = xn;
-        rd[i] = a * nwd * xn;
+        an[i] = a * nwd;
     }
-    const float rsum = reduce_scatter<kColTP, 32>(rd, lane);
+    const float rsum = reduce_scatter_dot<false>(xv, an, lane);
     if (lane % (kWave / kColTP) == 0) part[lane / (kWave / kColTP)][wave] = rsum;
     // d_res loads go out before the barrier, with the row sums in flight
     float dr[kColTP];
@@ -349,9 +349,10 @@ __global__ __launch_bounds__(kColsMaxD) void norm_conv_bwd_cols_kernel(
 // Bound by latency: 24 waves a CU, and a workgroup's loads, sums and stores one
 // after the other. A load masked as it arrives made every next one wait for it,
 // and 23 wave sums of six lane exchanges each were a third of the code; with the
-// loads asked for together and the rows summed in one halving (the same tree per
-// row) 32 x 512 positions of 768 channels take 29 us instead of 39 (100 MB, 21 us
-// at a copy's rate), 117 positions 9.5 instead of 12.7.
+// loads asked for together and the rows summed in one halving (reduce_scatter_dot,
+// which gives a row the bits of a wave sum by itself) 32 x 512 positions of 768
+// channels take 29 us instead of 39 (100 MB, 21 us at a copy's rate), 117
+// positions 9.5 instead of 12.7.
 template <typename TX, typename TO>
 __global__ __launch_bounds__(1024) void norm_conv_fwd_cols_kernel(const TX *__restrict__ x,
                                                                   const float *__restrict__ nw,
@@ -380,12 +381,12 @@ __global__ __launch_bounds__(1024) void norm_conv_fwd_cols_kernel(const TX *__re
 #pragma unroll
     for (int m = 0; m < W; ++m) xv[m] = (used(m) && vd) ? xv[m] : 0.f;
     {
-        float tile[kColTP], hl[kMaxTaps];   // the squares of the tile's rows, and of the halo's
+        float tile[kColTP], hl[kMaxTaps];   // the tile's rows, and the halo's
 #pragma unroll
-        for (int i = 0; i < kColTP; ++i) tile[i] = xv[halo + i] * xv[halo + i];
+        for (int i = 0; i < kColTP; ++i) tile[i] = xv[halo + i];
 #pragma unroll
-        for (int m = 0; m < kMaxTaps; ++m) hl[m] = m < halo ? xv[m] * xv[m] : 0.f;
-        const float st = reduce_scatter<kColTP, 32>(tile, lane), sh = reduce_scatter<kMaxTaps, 32>(hl, lane);
+        for (int m = 0; m < kMaxTaps; ++m) hl[m] = m < halo ? xv[m] : 0.f;
+        const float st = reduce_scatter_dot<true>(tile, tile, lane), sh = reduce_scatter_dot<true>(hl, hl, lane);
         if (lane % (kWave / kColTP) == 0) part[halo + lane / (kWave / kColTP)][wave] = st;
         if (lane % (kWave / kMaxTaps) == 0 && lane / (kWave / kMaxTaps) < halo) part[lane / (kWave / kMaxTaps)][wave] = sh;
     }

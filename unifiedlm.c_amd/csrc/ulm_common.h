@@ -88,6 +88,26 @@ template <int V, int MASK> __device__ __forceinline__ float reduce_scatter(float
     }
 }
 
+// Sums a[k] b[k] over the wave as reduce_scatter does, the products formed in the
+// first halving: a lower lane's product is added unrounded (fused) to the rounded
+// one of the lane 32 above, the sum that `v + __shfl_xor(v, 32)` of a product v
+// compiles to in lane 0's tree. So a row sums to the same bits here as in a
+// wave_sum by itself. SQUARE: b is a.
+template <bool SQUARE, int V> __device__ __forceinline__ float reduce_scatter_dot(float (&a)[V], float (&b)[V], int lane) {
+    static_assert(V > 1, "halves of the values");
+    float t[V / 2];
+#pragma unroll
+    for (int k = 0; k < V / 2; ++k) {
+        // the lower lanes' operands of value k (in the upper lanes: of k + V / 2), then the upper lanes'
+        const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(a[k]), __float_as_uint(a[k + V / 2]), false, false);
+        auto y = x;
+        if constexpr (!SQUARE)
+            y = __builtin_amdgcn_permlane32_swap(__float_as_uint(b[k]), __float_as_uint(b[k + V / 2]), false, false);
+        t[k] = __builtin_fmaf(__uint_as_float(x[0]), __uint_as_float(y[0]), __uint_as_float(x[1]) * __uint_as_float(y[1]));
+    }
+    return reduce_scatter<V / 2, 16>(t, lane);
+}
+
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
