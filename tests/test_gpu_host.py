@@ -133,3 +133,64 @@ def test_module_forward_under_autocast():
     ref = kernel.block_fwd(x, p.norm.weight, p.conv.weight, p.key.weight, p.key.bias, p.log_eps, p.val.weight,
                            p.mu.weight, p.log_rate, p.log_w, p.norm.eps, torch.bfloat16)[0]
     assert torch.equal(got, ref) and got.requires_grad
+
+
+def _block_leaves(bias=True):
+    args, dout = _args(2, 40, 32, 64, 4, 1, bias=bias)
+    return args, [a for a in args if a is not None], dout
+
+
+def _memory_leaves(parameter):
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    r = (torch.rand(2, 40, 96, device="cuda", generator=gen) / 96).requires_grad_(True)
+    v = torch.randn(2, 40, 64, device="cuda", generator=gen).requires_grad_(True)
+    g, w = torch.tensor(-0.05, device="cuda", requires_grad=True), torch.full((96,), 4.0, device="cuda")
+    return [r, v, g, torch.nn.Parameter(w) if parameter else w.requires_grad_(True)]
+
+
+@pytest.mark.parametrize("which", ["block", "block without bias", "memory", "memory with a Parameter"])
+def test_second_derivative_raises(which):
+    """create_graph gives the first gradients, the same bits, and a second backward is refused: no term of it may
+    vanish without an error."""
+    say(f"second derivatives of {which}")
+    if which.startswith("block"):
+        args, leaves, _ = _block_leaves("without" not in which)
+        call = lambda: kernel.unified_block(*args, 1e-5).square().sum()  # noqa: E731
+    else:
+        leaves = _memory_leaves("Parameter" in which)
+        call = lambda: sum(t.square().sum() for t in kernel.unified_memory(*leaves))  # noqa: E731
+    first = torch.autograd.grad(call(), leaves)
+    loss = call()
+    again = torch.autograd.grad(loss, leaves, create_graph=True)
+    assert all(a.requires_grad and torch.equal(a, b) for a, b in zip(again, first))
+    with pytest.raises(RuntimeError, match="no autograd formula"):
+        (loss + again[0].square().sum()).backward()
+
+
+@pytest.mark.parametrize("which", ["block", "block without bias", "memory", "memory, q alone"])
+def test_batch_of_gradients(which):
+    """is_grads_batched: the vmapped backward, against one backward for each gradient."""
+    say(f"a batch of gradients through {which}")
+    if which.startswith("block"):
+        args, leaves, dout = _block_leaves("without" not in which)
+        out = kernel.unified_block(*args, 1e-5)
+    else:
+        leaves = _memory_leaves(True)
+        out = kernel.unified_memory(*leaves)[0 if "alone" in which else 1]
+        leaves = leaves if "alone" not in which else [leaves[0], leaves[2], leaves[3]]
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    ups = torch.randn(3, *out.shape, device="cuda", generator=gen)
+    got = torch.autograd.grad(out, leaves, ups, is_grads_batched=True, retain_graph=True)
+    each = [torch.autograd.grad(out, leaves, u, retain_graph=True) for u in ups]
+    for a, b in zip(got, zip(*each)):
+        assert torch.equal(a, torch.stack(b))
+
+
+def test_gradient_with_a_negative_bit():
+    """A gradient that is a lazily negated view counts with its sign."""
+    say("a gradient with the negative bit")
+    args, leaves, dout = _block_leaves()
+    out = kernel.unified_block(*args, 1e-5)
+    got = torch.autograd.grad(out, leaves, torch._neg_view(dout), retain_graph=True)
+    ref = torch.autograd.grad(out, leaves, -dout)
+    assert all(torch.equal(a, b) for a, b in zip(got, ref))

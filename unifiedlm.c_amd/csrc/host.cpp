@@ -12,6 +12,7 @@
 // functorch transforms, forward-mode tangents, tensor subclasses, disagreeing
 // shapes, other dtypes and devices.
 #include <ATen/ATen.h>
+#include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/custom_function.h>
@@ -68,6 +69,7 @@ struct Maker {
 // keys of tensors, and of the thread, that only the Python implementations know how to meet
 const c10::DispatchKeySet kNotPlain({c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::FuncTorchBatched,
                                      c10::DispatchKey::FuncTorchVmapMode, c10::DispatchKey::Functionalize,
+                                     c10::DispatchKey::Batched, c10::DispatchKey::VmapMode,
                                      c10::DispatchKey::Python, c10::DispatchKey::PythonTLSSnapshot,
                                      c10::DispatchKey::Negative, c10::DispatchKey::Conjugate,
                                      c10::DispatchKey::ZeroTensor, c10::DispatchKey::Named});
@@ -76,6 +78,27 @@ bool plain_thread() {
     return !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) &&
            !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Python) &&
            !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Functionalize) && !torch::jit::tracer::isTracing();
+}
+
+// Whether a node's backward may launch on these gradients and saved tensors by
+// itself. Not where the backward is to be differentiated (create_graph), or where
+// a gradient, or what a saved-tensor hook gave back, is a batch of tensors or
+// another that only a dispatch can meet: the registered backward op serves those
+// as it does for a traced call, and has no derivative of its own, so that a
+// second one raises.
+bool launches(const variable_list &grads, const variable_list &saved) {
+    bool ok = !at::GradMode::is_enabled() && plain_thread();
+    for (const variable_list *list : {&grads, &saved})
+        for (const Tensor &t : *list) {
+            if (!t.defined()) continue;
+            TORCH_CHECK(t.device() == saved[0].device(), "tensors on different devices: ", saved[0].device(), " and ", t.device());
+            ok = ok && !t.key_set().has_any(kNotPlain) && t.layout() == at::kStrided;
+        }
+    return ok;
+}
+
+template <class F> auto registered(const char *name) {
+    return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<F>();
 }
 
 // a Tensor or Parameter proper (no subclass), strided, on a GPU, floating, with no tangent; undefined otherwise
@@ -102,7 +125,7 @@ struct FM : torch::autograd::Function<FM> {
         check("ulm_fm_fwd", ulm_fm_fwd(fp(r32), vc.data_ptr(), vdt, fp(g1), fp(w32), fpm(q), fast.data_ptr(), vdt,
                                        saved.data_ptr(), sb, ws.data_ptr(), wb, B, T, A, D, stream_of(r)));
         ctx->save_for_backward({r, g, w, saved});
-        ctx->saved_data["vdt"] = static_cast<int64_t>(vdt);
+        ctx->saved_data["vdt"] = static_cast<int64_t>(v.scalar_type());
         ctx->saved_data["D"] = static_cast<int64_t>(D);
         ctx->set_materialize_grads(false);
         return {q, fast};
@@ -113,10 +136,19 @@ struct FM : torch::autograd::Function<FM> {
         const Tensor dq = grads[0];
         Tensor dfast = grads[1];
         if (!dq.defined() && !dfast.defined()) return {Tensor(), Tensor(), Tensor(), Tensor()};
-        at::AutoDispatchBelowAutograd guard;
         const int B = r.size(0), T = r.size(1), A = r.size(2), D = ctx->saved_data["D"].toInt();
-        const int vdt = ctx->saved_data["vdt"].toInt();
+        const auto vt = static_cast<at::ScalarType>(ctx->saved_data["vdt"].toInt());
+        const int vdt = code(vt);
         const Maker make(r);
+        if (!launches(grads, sv)) {
+            using F = std::tuple<Tensor, Tensor, Tensor, Tensor>(const Tensor &, const Tensor &, const Tensor &, const Tensor &,
+                                                                 at::ScalarType, const std::optional<Tensor> &, const Tensor &);
+            if (!dfast.defined()) dfast = at::zeros({B, T, D}, make.opt.dtype(at::kFloat));
+            const auto [dr, dv, dg, dw] = registered<F>("ulm::fm_bwd").call(
+                r, g, w, saved, vt, dq.defined() ? std::optional<Tensor>(dq) : std::nullopt, dfast);
+            return {dr, dv, dg.reshape(g.sizes()), dw};
+        }
+        at::AutoDispatchBelowAutograd guard;
         dfast = dfast.defined() ? dfast.contiguous() : at::zeros({B, T, D}, make.opt.dtype(at::kFloat));
         const int ddt = code(dfast.scalar_type());
         const Tensor r32 = f32c(r), g1 = f32c(g), w32 = f32c(w), dqo = dq.defined() ? f32c(dq) : dq;
@@ -244,6 +276,17 @@ struct BlockFn : torch::autograd::Function<BlockFn> {
                      &val_w = sv[6], &mu_w = sv[7], &log_rate = sv[8], &log_w = sv[9], &rstd = sv[10], &h = sv[11],
                      &u = sv[12], &pre = sv[13], &denom = sv[14], &g1 = sv[15], &w32 = sv[16], &saved = sv[17],
                      &qw = sv[18];
+        if (!launches(grads, sv)) {
+            using T1 = const Tensor &;
+            using F = std::tuple<Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor, Tensor>(
+                T1, T1, T1, T1, T1, const std::optional<Tensor> &, T1, T1, T1, T1, T1, T1, T1, T1, T1, T1, T1, T1, T1, T1,
+                at::ScalarType);
+            const std::optional<Tensor> bias = key_b.defined() ? std::optional<Tensor>(key_b) : std::nullopt;
+            auto [dx, dnw, dcw, dkey, dbias, dle, dval, dmu, dlr, dlw] = registered<F>("ulm::block_bwd").call(
+                grads[0], x, norm_w, conv_w, key_w, bias, log_eps, val_w, mu_w, log_rate, log_w, rstd, h, u, pre, denom, g1,
+                w32, saved, qw, static_cast<at::ScalarType>(ctx->saved_data["cdt"].toInt()));
+            return {dx, dnw, dcw, dkey, bias ? dbias : Tensor(), dle, dval, dmu, dlr, dlw, Tensor(), Tensor()};
+        }
         at::AutoDispatchBelowAutograd guard;
         c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
         const auto cdt = static_cast<at::ScalarType>(ctx->saved_data["cdt"].toInt());
