@@ -107,3 +107,17 @@ def test_final_norm_in_one_launch():
         lm.norm.register_forward_hook(lambda m, i, o: seen.append(o))
         lm.step(torch.zeros(2, dtype=torch.long, device="cuda"), lm.init_states(2, "cuda"))
     assert len(seen) == 1
+
+
+@pytest.mark.parametrize("form", [tuple, iter, lambda states: dict(enumerate(states)).values()])
+def test_states_in_any_iterable(form):
+    """UnifiedLM.step takes its states from any iterable, and no more of them than it has blocks."""
+    lm = _block(96, 140, 4, 5, n_layers=3)
+    say("UnifiedLM.step: states in a tuple, an iterator, a view")
+    a, b = lm.init_states(2, "cuda"), lm.init_states(2, "cuda")
+    for t in range(3):
+        tokens = torch.tensor([t, t + 1], device="cuda")
+        assert torch.equal(lm.step(tokens, form(a)), lm.step(tokens, b))
+    more = iter(a + ["left"])
+    lm.step(tokens, more)
+    assert next(more) == "left"

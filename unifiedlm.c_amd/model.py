@@ -362,10 +362,11 @@ class UnifiedLM(nn.Module):
     def step(self, tokens: torch.Tensor, states) -> torch.Tensor:
         """One position for a batch of sequences: tokens (B,) -> logits (B, V)."""
         h = self.tok_embeddings(tokens)
-        out = self._few_steps(h, states)
+        pairs = list(zip(self.layers, states))   # states: any iterable
+        out = self._few_steps(h, pairs)
         if out is not None:
             return self.output(self._final_norm(out))
-        for layer, s in zip(self.layers, states):
+        for layer, s in pairs:
             h = layer.step(h, s)
         return self.output(self.norm(h))
 
@@ -379,21 +380,21 @@ class UnifiedLM(nn.Module):
                 return out
         return norm(h)
 
-    def _few_steps(self, h, states):
+    def _few_steps(self, h, pairs):
         """Every block's step in one native call (kernel.decode_step), or None
         where a block would not take it by itself: other dtypes, large states,
         slot counts without the deferred state, steps of a
         subclass's own."""
-        if h.dtype != torch.float32 or len(states) != len(self.layers):
+        if h.dtype != torch.float32 or not pairs:
             return None
-        for layer, s in zip(self.layers, states):
+        for layer, s in pairs:
             if type(layer) is not UnifiedBlock or "step" in layer.__dict__:
                 return None
             slots = s["S"].shape[-1]
             if slots % 4 or slots > 4096:
                 return None
             layer._pending(s, h.device)
-        return _few_step(h, self.layers, states) if states else None
+        return _few_step(h, *map(list, zip(*pairs)))
 
     @torch.no_grad()
     def decode_greedy(self, prompt: torch.Tensor, steps: int, prefill: bool = True) -> torch.Tensor:
