@@ -367,8 +367,8 @@ int ulm_decode_flush(float *S, const float *pv, const float *pr, int m, const fl
  * conv_buf (N,D,Kc-1), S (N,D,A) = S_base, c (N,A) and r_prev (N,A), updated in
  * place, and the pending values pv (16,N,D) and keys pr (16,N,A), of which
  * `pending` (0 .. 15) are held. The position appends one; a block that held 15
- * is written back and holds none afterwards. mu_w, w, S, c and r_prev 16-byte
- * aligned; A % 4 == 0, A <= 4096, Kc <= 8. Workspace of
+ * is written back and holds none afterwards. mu_w, w, S, c, r_prev and pr
+ * 16-byte aligned; A % 4 == 0, A <= 4096, Kc <= 8. Workspace of
  * ulm_decode_step_workspace_bytes() bytes (0: sizes this form does not take). */
 typedef struct ulm_decode_layer {
     const float *norm_w, *conv_w, *key_w, *key_b, *log_eps, *val_w, *mu_w, *w, *g;

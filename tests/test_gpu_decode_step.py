@@ -121,3 +121,27 @@ def test_states_in_any_iterable(form):
     more = iter(a + ["left"])
     lm.step(tokens, more)
     assert next(more) == "left"
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("where,key,change", [
+    ("state", "pr", "misaligned"), ("state", "S", "misaligned"), ("state", "S", "subclass"), ("state", "c", "negative"),
+    ("params", "w", "negative"), ("params", "mu_w", "subclass"), ("params", "mu_w", "misaligned")])
+def test_tensors_left_to_the_per_kernel_form(where, key, change):
+    """Tensors off 16 bytes, subclasses and lazily negated ones: nothing is touched."""
+    say(f"the two-launch step leaves a {change} {key} of the {where} alone")
+    block = _block(64, 128, 4, 1).layers[0]
+    s = block.init_state(3, torch.device("cuda"))
+    block._pending(s, torch.device("cuda"))
+    held = s if where == "state" else s["params"]
+    t = held[key]
+    if change == "misaligned":
+        held[key] = torch.zeros(t.numel() + 1, device="cuda")[1:].view(t.shape).copy_(t)
+    else:
+        held[key] = t.as_subclass(_Sub) if change == "subclass" else torch._neg_view(t)
+    before = {k: s[k].detach().clone() for k in ("S", "c", "r_prev", "buf")}
+    assert model_mod.decode_step(torch.randn(3, 64, device="cuda"), [s], [1e-5]) is None
+    assert s["np"] == 0 and all(torch.equal(s[k], t) for k, t in before.items())

@@ -506,9 +506,9 @@ extern "C" int ulm_decode_step(const ulm_decode_layer *layers, int n_layers, con
                     static_cast<long long>(l.pending));
         for (const void *p : {static_cast<const void *>(l.mu_w), static_cast<const void *>(l.w),
                               static_cast<const void *>(l.S), static_cast<const void *>(l.c),
-                              static_cast<const void *>(l.r_prev)})
+                              static_cast<const void *>(l.r_prev), static_cast<const void *>(l.pr)})   // pr: the write-back's
             ULM_REQUIRE(reinterpret_cast<uintptr_t>(p) % 16 == 0,
-                        "ulm_decode_step: layer %d: mu_w, w, S, c and r_prev must be 16-byte aligned", i);
+                        "ulm_decode_step: layer %d: mu_w, w, S, c, r_prev and pr must be 16-byte aligned", i);
     }
     hipStream_t s = static_cast<hipStream_t>(stream);
     for (int i = 0; i < n_layers; ++i) {

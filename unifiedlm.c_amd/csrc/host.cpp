@@ -442,10 +442,10 @@ py::object decode_step(const py::handle &x_, const py::list &states, const py::l
         if (!p || !PyDict_Check(p)) return py::none();
         auto get = [&](PyObject *d, const py::str &key) -> const at::TensorImpl * {
             PyObject *o = PyDict_GetItem(d, key.ptr());
-            if (!o || !THPVariable_Check(o)) return nullptr;
+            if (!o || !THPVariable_CheckExact(o)) return nullptr;
             const Tensor &t = THPVariable_Unpack(o);
             return t.defined() && t.is_cuda() && t.scalar_type() == at::kFloat && t.device() == x.device() &&
-                           t.layout() == at::kStrided && t.is_contiguous()
+                           t.layout() == at::kStrided && t.is_contiguous() && !t.key_set().has_any(kNotPlain)
                        ? t.unsafeGetTensorImpl()
                        : nullptr;
         };
@@ -464,8 +464,8 @@ py::object decode_step(const py::handle &x_, const py::list &states, const py::l
             const at::TensorImpl *t = j < 9 ? get(p, keys.param[j]) : get(s, keys.state[j - 9]);
             if (!t || t->sizes() != at::IntArrayRef(shapes[j])) return py::none();
             at[j] = const_cast<void *>(t->data());
-            // mu_w, w, S, c, r_prev: 16-byte accesses
-            if ((j == 6 || j == 7 || (j >= 10 && j <= 12)) && reinterpret_cast<uintptr_t>(at[j]) % 16) return py::none();
+            // mu_w, w, S, c, r_prev, pr: 16-byte accesses
+            if ((j == 6 || j == 7 || (j >= 10 && j <= 12) || j == 14) && reinterpret_cast<uintptr_t>(at[j]) % 16) return py::none();
         }
         PyObject *m = PyDict_GetItem(s, keys.np.ptr());
         const long held = m && PyLong_Check(m) ? PyLong_AsLong(m) : -1;
