@@ -1062,8 +1062,12 @@ __device__ __forceinline__ void pair_small_body(const Args &p, const int bid) {
             const float x = acc[r];
             X[(8 * (r / 4) + 4 * h + r % 4) * XS + lc] = x;
         }
-        __builtin_amdgcn_s_waitcnt(kWaitLgkm0);   // the tile's one wave: its writes before its reads
+        // the tile's one wave: its lanes' writes before its other lanes' reads, for the compiler (the fences) and in
+        // the LDS queue
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
         __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
     const float g = p.g[0];
     const bool want_t = p.pout_t != nullptr;
