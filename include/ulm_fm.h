@@ -357,7 +357,8 @@ int ulm_decode_flush(float *S, const float *pv, const float *pr, int m, const fl
                      const float *x, const float *ymu, float *out, int N, int D, int A, void *stream);
 
 /* One position of n_layers consecutive blocks for up to 256 sequences whose
- * states are small (up to 320 MB per block), two launches per block (a third
+ * states are small (up to 320 MB per block, and less for many sequences:
+ * ulm_decode_step_workspace_bytes() tells), two launches per block (a third
  * where a block's 16th term makes it write its state back): what the per-kernel entries above and the three projections
  * compute, on the same deferred state. x (N,D) is the first block's input,
  * out (N,D) the last one's output, neither aliasing the other.

@@ -40,10 +40,20 @@ def test_refuses_null_pointers_and_full_states(change):
 
 
 def test_sizes():
-    """Up to 320 MB of state per block, 256 sequences, 4096 slots in fours, 8 taps, features whose row fits 60 KB."""
+    """Up to 256 sequences, 4096 slots in fours, 8 taps, features whose row fits 60 KB."""
     takes = lambda *s: nat.lib().ulm_decode_step_workspace_bytes(*s) > 0  # noqa: E731
-    assert takes(80, 1024, 1024, 4) and not takes(80, 1024, 1028, 4)   # 320 MB of S_base, and past it
     assert takes(256, 64, 128, 4) and not takes(257, 64, 128, 4)
     assert takes(1, 64, 4096, 4) and not takes(1, 64, 4100, 4) and not takes(1, 64, 126, 4)
     assert takes(1, 64, 128, 8) and not takes(1, 64, 128, 9) and takes(1, 64, 128, 1)
     assert takes(1, 15360, 4, 4) and not takes(1, 15361, 4, 4)
+
+
+@pytest.mark.parametrize("N,D,A,taken", [
+    (256, 64, 128, True), (256, 64, 1024, True), (128, 288, 712, True), (16, 768, 3072, True), (32, 768, 3072, True),
+    (40, 512, 3072, True), (1, 288, 712, True), (8, 768, 3072, True),
+    (64, 768, 3072, False), (48, 768, 2048, False), (256, 288, 712, False), (128, 768, 768, False),
+    (256, 512, 512, False), (256, 768, 128, False), (256, 64, 4096, False), (256, 32, 4096, False), (100, 1600, 400, False),
+])
+def test_takes_the_sizes_it_is_faster_at(N, D, A, taken):
+    """Both sides of the line between this form and the per-kernel one, by what each took there."""
+    assert (nat.lib().ulm_decode_step_workspace_bytes(N, D, A, 4) > 0) == taken

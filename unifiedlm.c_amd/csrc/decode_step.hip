@@ -1,7 +1,8 @@
 // One decode position of consecutive blocks, two launches per block:
 // UnifiedBlock.step (model.py:96-111, run.c:193-265) on the deferred state of
 // decode.hip (S_base and up to kMaxPending pending terms), for batches whose
-// state is small (kMaxState).
+// position takes two launches less time than it takes the host to enqueue the
+// per-kernel form's (kMaxCost).
 //
 // There a position is bound by launches and memory latency, not by bytes: the
 // per-kernel form (RMSNorm + conv, three GEMMs, address, state read: 6 launches
@@ -34,10 +35,18 @@ namespace step {
 
 constexpr int kMaxPending = 16;   // as decode.hip
 constexpr int kMaxN = 256;        // sequences
-// bytes of S_base up to which this form is the faster one: at the 110M widths 16 positions of a block took 1.34 ms
-// against 1.65 at 32 sequences (302 MB), and 2.50 against 2.32 at 64, where the per-kernel form's state read (7 TB/s
-// against 4.5 here, which walks several sequences' rows and mu's at once) outweighs its other launches
-constexpr size_t kMaxState = 320u << 20;
+constexpr size_t kMaxState = 320u << 20;   // bytes of S_base
+// Microseconds up to which a block's position takes this form (cost below): the
+// per-kernel form's eight calls take 88 of host time, whatever their sizes, and
+// from about 250 MB of state on 94 of the device's. 16 positions of one block, us,
+// this form / per kernel, at (sequences, features, slots) and the cost:
+//   (256, 64, 128)     27    405 / 1440        (26, 768, 4096)    92   1656 / 1635
+//   (16, 768, 3072)    52    898 / 1421        (48, 768, 2048)    99   1539 / 1498
+//   (256, 64, 1024)    54    825 / 1418        (256, 288, 712)   108   1731 / 1450
+//   (128, 288, 712)    61    913 / 1422        (128, 768, 768)   141   2146 / 1452
+//   (40, 512, 3072)    80   1359 / 1433        (256, 512, 512)   153   2436 / 1445
+//   (32, 768, 3072)    90   1330 / 1504        (256, 768, 400)   210   3520 / 1781
+constexpr double kMaxCost = 92;
 constexpr int kWgN = 16;          // sequences per workgroup of the first phase
 constexpr int kLdsFloats = 15 * 1024;   // of dynamic LDS per workgroup: 60 KB
 constexpr int kRows = 4;          // weight rows per wave
@@ -443,6 +452,14 @@ int launch_in(const Layer &L, const float *x, const Ws &ws, int N, int D, int A,
     return check_launch("decode_in_kernel");
 }
 
+// A position's microseconds in this form, within 10% where it is near the line
+// (30 shapes, 1 to 256 sequences, 16 to 2048 features, 64 to 4096 slots): two
+// launches; S_base, mu and the key rows; the value rows; z, c and the pending
+// keys, several passes of N A floats; and h and u, which every workgroup of the
+// first phase forms for itself, with what a wave of the second one does per
+// feature before it walks the slots.
+double cost(double N, double D, double A) { return 14 + 1e-6 * N * (0.70 * D * A + 0.185 * D * D + 75 * A + 540 * D); }
+
 // sequences per workgroup of the first phase, their u in LDS: evenly over the fewest groups of at most kWgN
 int in_groups(int N, int D) {
     const int most = std::min(kWgN, kLdsFloats / D);
@@ -482,7 +499,7 @@ using namespace ulm;
 // the shapes this form takes; at least one sequence's u fits the LDS of a workgroup
 static bool step_supported(int N, int D, int A, int Kc) {
     return N >= 1 && N <= step::kMaxN && D >= 1 && A >= 4 && A % 4 == 0 && A <= 4096 && Kc >= 1 && Kc <= step::kMaxTaps &&
-           step::in_groups(N, D) > 0 && 4ull * N * D * A <= step::kMaxState;
+           step::in_groups(N, D) > 0 && 4ull * N * D * A <= step::kMaxState && step::cost(N, D, A) <= step::kMaxCost;
 }
 
 extern "C" size_t ulm_decode_step_workspace_bytes(int N, int D, int A, int Kc) {
