@@ -413,6 +413,28 @@ py::object prefill(double eps, at::ScalarType cdt, const py::args &args) {
     return py::make_tuple(y.view({B, T, D}), S, c, r_prev, buf, k.g1, k.w32);
 }
 
+// fp32 copies of tensors, one allocation and one launch, or None (UnifiedBlock._step_params' matrices)
+py::object copies(const py::args &args) {
+    if (!plain_thread()) return py::none();
+    at::NoGradGuard no_grad;
+    at::AutoDispatchBelowAutograd guard;
+    std::vector<Tensor> flat, out;
+    for (const auto &a : args) {
+        const Tensor t = plain(a);
+        if (!t.defined()) return py::none();
+        out.push_back(t);
+        flat.push_back(f32c(t).view(-1));
+    }
+    const Tensor all = at::cat(flat);
+    int64_t from = 0;
+    for (Tensor &t : out) {
+        const int64_t n = t.numel();
+        t = all.narrow(0, from, n).view(t.sizes());
+        from += n;
+    }
+    return py::cast(out);
+}
+
 // ---- decode positions (kernel.decode_step)
 
 // the state dicts' keys, made once
@@ -489,5 +511,6 @@ PYBIND11_MODULE(ulm_host, m) {
     m.def("memory", &memory);
     m.def("block", &block);
     m.def("prefill", &prefill);
+    m.def("copies", &copies);
     m.def("decode_step", &decode_step);
 }

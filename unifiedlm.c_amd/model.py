@@ -30,7 +30,7 @@ import torch.nn.functional as F
 
 from kernel import (CHUNK, LOG_W_MAX, LOG_W_MIN, block_eager, block_prefill, block_prefill_eager, decode_addr,
                     decode_addr_deferred, decode_deferred, decode_pre, decode_state, decode_step, fm_prefill,
-                    relu2_address, rms_norm, unified_block, unified_memory)
+                    matrix_copies, relu2_address, rms_norm, unified_block, unified_memory)
 
 # whether any hook is registered for every module (assumed where torch does not say)
 _any_global_hook = getattr(nn.modules.module, "_has_any_global_hook", lambda: True)
@@ -154,15 +154,19 @@ class UnifiedBlock(nn.Module):
 
     @torch.no_grad()
     def _step_params(self, device, w=None, g=None):
-        """What every step reads, in contiguous fp32 (the parameters themselves
-        where they are that already), taken once per decode session: weights
-        do not change while it decodes."""
+        """What every step reads, in contiguous fp32, taken once per decode
+        session: weights do not change while it decodes. The key, value and mu
+        matrices are copies, as the prior mass and the decay are values of this
+        moment, so that a session goes on with them whatever becomes of the
+        module's; the small rest is the parameters themselves where they are
+        contiguous fp32."""
         def f32(t):
             return t.detach().to(device=device, dtype=torch.float32).contiguous()
+        key_w, mu_w, val_w = matrix_copies(device, self.key.weight, self.mu.weight, self.val.weight)
         return {"norm_w": f32(self.norm.weight), "conv_w": f32(self.conv.weight[:, 0, :]),
-                "key_w": f32(self.key.weight), "key_b": f32(self.key.bias),
-                "log_eps": f32(self.log_eps).reshape(1), "val_w": f32(self.val.weight),
-                "mu_w": f32(self.mu.weight), "w": f32(self._w()) if w is None else w,
+                "key_w": key_w, "key_b": f32(self.key.bias),
+                "log_eps": f32(self.log_eps).reshape(1), "val_w": val_w,
+                "mu_w": mu_w, "w": f32(self._w()) if w is None else w,
                 "g": f32(self._decay_log()).reshape(1) if g is None else g}
 
     @torch.no_grad()
