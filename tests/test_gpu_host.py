@@ -194,3 +194,53 @@ def test_gradient_with_a_negative_bit():
     got = torch.autograd.grad(out, leaves, torch._neg_view(dout), retain_graph=True)
     ref = torch.autograd.grad(out, leaves, -dout)
     assert all(torch.equal(a, b) for a, b in zip(got, ref))
+
+
+@pytest.mark.parametrize("which", ["memory", "block", "prefill", "copies", "decode_step"])
+def test_other_threads_run_during_a_call(which):
+    """The interpreter's lock is free while a call works: with no forced switch for 1000 s, a thread that waits for
+    the lock gets it inside one of the calls or never."""
+    import sys
+    import threading
+    import time
+    say(f"another thread runs during {which}")
+    host = nat.host()
+    args, _ = _args(2, 300, 96, 128, 4, 3)
+    args = [a.detach() for a in args]
+    if which == "memory":
+        leaves = [t.detach() for t in _memory_leaves(False)]
+        call = lambda: host.memory(*leaves)  # noqa: E731
+    elif which == "copies":
+        call = lambda: host.copies(args[3], args[7], args[6])  # noqa: E731
+    elif which == "decode_step":
+        block = UnifiedBlock(ModelArgs(dim=64, hidden_dim=128)).cuda()
+        s = block.init_state(2, torch.device("cuda"))
+        block._pending(s, torch.device("cuda"))
+        x = torch.randn(2, 64, device="cuda")
+        call = lambda: host.decode_step(x, [s], [1e-5])  # noqa: E731
+    else:
+        call = lambda: getattr(host, which)(1e-5, torch.float32, *args)  # noqa: E731
+    assert call() is not None
+    torch.cuda.synchronize()
+    ran, kept, gate = [], [], threading.Lock()
+    gate.acquire()
+
+    def other():
+        with gate:
+            ran.append(True)
+    thread = threading.Thread(target=other)
+    thread.start()
+    time.sleep(0.1)   # it waits at the gate
+    before = sys.getswitchinterval()
+    sys.setswitchinterval(1000)
+    try:
+        gate.release()
+        for _ in range(2000):
+            kept.append(call())   # dropping a tensor frees the lock for a moment by itself
+            if ran:
+                break
+        seen = bool(ran)
+    finally:
+        sys.setswitchinterval(before)
+    thread.join()
+    assert seen

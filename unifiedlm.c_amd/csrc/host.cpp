@@ -6,11 +6,12 @@
 // host time for 283 us of GPU work (8 x 200 positions of the default model's
 // widths in fp32), and takes about 390 us from here. The prefill of one prompt
 // of 117 positions at the 110M widths went 238 -> 143 us, a decode position of
-// the default model 244 -> 171 us. Everything here evaluates what kernel.py's implementations evaluate,
-// with the same native calls in the same order; a call that is not a plain eager
-// one, or that they would refuse, returns None and is left to them: tracing,
-// functorch transforms, forward-mode tangents, tensor subclasses, disagreeing
-// shapes, other dtypes and devices.
+// the default model 244 -> 171 us. Everything here evaluates what kernel.py's
+// implementations evaluate, with the same native calls in the same order, and
+// without the interpreter's lock; a call that is not a plain eager one, or that
+// they would refuse, returns None and is left to them: tracing, functorch
+// transforms, forward-mode tangents, tensor subclasses, disagreeing shapes, other
+// dtypes and devices.
 #include <ATen/ATen.h>
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
@@ -101,6 +102,12 @@ template <class F> auto registered(const char *name) {
     return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<F>();
 }
 
+// f() without the interpreter's lock: launches, library GEMMs and the allocator may wait, and other threads run
+template <class F> auto unlocked(F f) {
+    py::gil_scoped_release release;
+    return f();
+}
+
 // a Tensor or Parameter proper (no subclass), strided, on a GPU, floating, with no tangent; undefined otherwise
 Tensor plain(const py::handle &h) {
     if (!THPVariable_CheckExact(h.ptr())) return {};
@@ -171,7 +178,7 @@ py::object memory(const py::handle &r_, const py::handle &v_, const py::handle &
         return py::none();
     for (const Tensor *t : {&v, &g, &w})
         if (t->device() != r.device()) return py::none();
-    const auto out = FM::apply(r, v, g, w);
+    const auto out = unlocked([&] { return FM::apply(r, v, g, w); });
     return py::make_tuple(py::cast(out[0]), py::cast(out[1]));
 }
 
@@ -377,17 +384,15 @@ bool gemm_dtype(at::ScalarType dt) { return dt == at::kFloat || dt == at::kBFloa
 py::object block(double eps, at::ScalarType cdt, const py::args &args) {
     const BlockArgs a(args);
     if (!a.ok || !gemm_dtype(cdt)) return py::none();
-    return py::cast(BlockFn::apply(a.x, a.norm_w, a.conv_w, a.key_w, a.key_b, a.log_eps, a.val_w, a.mu_w, a.log_rate, a.log_w,
-                                   eps, static_cast<int64_t>(cdt)));
+    return py::cast(unlocked([&] {
+        return BlockFn::apply(a.x, a.norm_w, a.conv_w, a.key_w, a.key_b, a.log_eps, a.val_w, a.mu_w, a.log_rate, a.log_w, eps,
+                              static_cast<int64_t>(cdt));
+    }));
 }
 
 // (out, S, c, r_prev, conv window, g, w) of kernel.block_prefill and UnifiedBlock.prefill; under no_grad
-py::object prefill(double eps, at::ScalarType cdt, const py::args &args) {
-    const BlockArgs a(args);
-    if (!a.ok || !gemm_dtype(cdt)) return py::none();
+std::vector<Tensor> prefill_of(const BlockArgs &a, double eps, at::ScalarType cdt, size_t wb) {
     const int B = a.x.size(0), T = a.x.size(1), D = a.x.size(2), A = a.key_w.size(0);
-    const size_t wb = ulm_block_fm_prefill_workspace_bytes(B, T, A, D, code(cdt));
-    if (wb == 0) return py::none();
     at::NoGradGuard no_grad;
     at::AutoDispatchBelowAutograd guard;
     c10::impl::ExcludeDispatchKeyGuard no_autocast(c10::autocast_dispatch_keyset);
@@ -410,29 +415,38 @@ py::object prefill(double eps, at::ScalarType cdt, const py::args &args) {
     const int kw = k.Kc - 1, n = std::min(kw, T);
     Tensor buf = n < kw ? at::zeros({B, D, kw}, k.make.opt.dtype(at::kFloat)) : k.make({B, D, kw});
     if (n > 0) buf.narrow(2, kw - n, n).copy_(k.h.narrow(1, T - n, n).transpose(1, 2));
-    return py::make_tuple(y.view({B, T, D}), S, c, r_prev, buf, k.g1, k.w32);
+    return {y.view({B, T, D}), S, c, r_prev, buf, k.g1, k.w32};
+}
+
+py::object prefill(double eps, at::ScalarType cdt, const py::args &args) {
+    const BlockArgs a(args);
+    if (!a.ok || !gemm_dtype(cdt)) return py::none();
+    const size_t wb = ulm_block_fm_prefill_workspace_bytes(a.x.size(0), a.x.size(1), a.key_w.size(0), a.x.size(2), code(cdt));
+    if (wb == 0) return py::none();
+    return py::tuple(py::cast(unlocked([&] { return prefill_of(a, eps, cdt, wb); })));
 }
 
 // fp32 copies of tensors, one allocation and one launch, or None (UnifiedBlock._step_params' matrices)
 py::object copies(const py::args &args) {
     if (!plain_thread()) return py::none();
-    at::NoGradGuard no_grad;
-    at::AutoDispatchBelowAutograd guard;
-    std::vector<Tensor> flat, out;
+    std::vector<Tensor> mats;
     for (const auto &a : args) {
-        const Tensor t = plain(a);
-        if (!t.defined()) return py::none();
-        out.push_back(t);
-        flat.push_back(f32c(t).view(-1));
+        mats.push_back(plain(a));
+        if (!mats.back().defined()) return py::none();
     }
-    const Tensor all = at::cat(flat);
-    int64_t from = 0;
-    for (Tensor &t : out) {
-        const int64_t n = t.numel();
-        t = all.narrow(0, from, n).view(t.sizes());
-        from += n;
-    }
-    return py::cast(out);
+    return py::cast(unlocked([&] {
+        at::NoGradGuard no_grad;
+        at::AutoDispatchBelowAutograd guard;
+        std::vector<Tensor> flat, out;
+        for (const Tensor &t : mats) flat.push_back(f32c(t).view(-1));
+        const Tensor all = at::cat(flat);
+        int64_t from = 0;
+        for (const Tensor &t : mats) {
+            out.push_back(all.narrow(0, from, t.numel()).view(t.sizes()));
+            from += t.numel();
+        }
+        return out;
+    }));
 }
 
 // ---- decode positions (kernel.decode_step)
@@ -496,10 +510,13 @@ py::object decode_step(const py::handle &x_, const py::list &states, const py::l
         layers[i] = ulm_decode_layer{f(0), f(1), f(2), f(3), f(4), f(5), f(6), f(7), f(8), f(9), f(10), f(11), f(12), f(13),
                                      f(14), eps[i].cast<double>(), held};
     }
-    at::NoGradGuard no_grad;
-    const Tensor out = at::empty_like(x), ws = Maker(x).bytes(wb);
-    check("ulm_decode_step", ulm_decode_step(layers.data(), layers.size(), fp(x), fpm(out), ws.data_ptr(), wb, N, D, A, Kc,
-                                             stream_of(x)));
+    const Tensor out = unlocked([&] {
+        at::NoGradGuard no_grad;
+        const Tensor y = at::empty_like(x), ws = Maker(x).bytes(wb);
+        check("ulm_decode_step", ulm_decode_step(layers.data(), layers.size(), fp(x), fpm(y), ws.data_ptr(), wb, N, D, A, Kc,
+                                                 stream_of(x)));
+        return y;
+    });
     for (size_t i = 0; i < layers.size(); ++i)
         states[i][keys.np] = py::int_((layers[i].pending + 1) % J);
     return py::cast(out);
