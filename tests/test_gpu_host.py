@@ -244,3 +244,23 @@ def test_other_threads_run_during_a_call(which):
         sys.setswitchinterval(before)
     thread.join()
     assert seen
+
+
+def test_function_modes_see_the_registered_op():
+    """A torch function mode sees the block's op, as without the host module; a default device is none."""
+    from torch.overrides import TorchFunctionMode
+    say("a block under a torch function mode and under a default device")
+    args, _ = _args(2, 40, 32, 64, 4, 1)
+    seen = []
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, a=(), kw=None):
+            seen.append(str(func))
+            return func(*a, **(kw or {}))
+    ref = kernel.block_eager(*args, 1e-5, torch.float32)
+    with Mode():
+        assert kernel.block_eager(*args, 1e-5, torch.float32) is None
+        got = kernel.unified_block(*args, 1e-5)
+    assert "ulm.block_fwd.default" in seen and torch.equal(got, ref)
+    with torch.device("cuda"):
+        assert kernel.block_eager(*args, 1e-5, torch.float32) is not None

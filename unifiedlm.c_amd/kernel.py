@@ -19,6 +19,7 @@ kernels used by UnifiedBlock.step.
 from typing import Optional
 
 import torch
+from torch.utils._device import DeviceContext
 
 import ulm_native as nat
 from ulm_native import call, ptr
@@ -152,15 +153,22 @@ torch.library.register_autograd("ulm::fm_fwd", _fm_backward, setup_context=_fm_s
 
 # the number of active torch dispatch modes (one assumed where torch does not say)
 _dispatch_modes = getattr(torch._C, "_len_torch_dispatch_stack", lambda: 1)
+_function_modes = getattr(torch._C, "_len_torch_function_stack", lambda: 1)
+
+
+def _watched():
+    """Whether a torch function mode, other than a default device, would see the registered ops' calls."""
+    modes = getattr(torch.overrides, "_get_current_function_mode_stack", lambda: [None])()
+    return any(type(m) is not DeviceContext for m in modes)
 
 
 def _plain_eager(*tensors):
     """True when the call runs eagerly on plain tensors: no torch.compile
-    trace, no dispatch mode (fake tensors, functionalization), and tensors or
-    parameters proper. The host module then takes it, without the registered
+    trace, no dispatch mode (fake tensors, functionalization), no function mode
+    that would see the call, and tensors or parameters proper. The host module then takes it, without the registered
     ops' dispatch and Python between the launches; the registered ops serve
     the rest (the module itself looks at the tensors it is given)."""
-    if torch.compiler.is_compiling() or _dispatch_modes() > 0:
+    if torch.compiler.is_compiling() or _dispatch_modes() > 0 or (_function_modes() > 0 and _watched()):
         return False
     return all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in tensors)
 
