@@ -10,7 +10,9 @@ from helpers import say
 
 pytestmark = pytest.mark.gpu
 
+import ulm_native as nat  # noqa: E402
 from kernel import unified_memory  # noqa: E402
+from ulm_native import call, ptr  # noqa: E402
 
 
 def _q64(r, lam, w):
@@ -61,3 +63,61 @@ def test_prior_masses_at_the_ends_of_the_range():
     got, want = q[0, T - 1].cpu(), (r[0, T - 1] / w).cpu()
     assert torch.equal(got, want), (got, want)
     assert torch.equal(q[0, :T - 1, :4], torch.zeros(T - 1, 4, device="cuda"))
+
+
+# ---- the address formed from pre (the fused block's input kind), w q out, the prefill's c and decayed keys
+
+def _block_rows(pre, bias, denom, v, g, w, x, prefill):
+    """(w q, x + fast[, S, c]) of ulm_block_fm_fwd or ulm_block_fm_prefill."""
+    (B, T, A), D = pre.shape, v.shape[-1]
+    dt, lib = nat.dtype_code(pre.dtype), nat.lib()
+    qw, y = torch.empty_like(pre), torch.empty(B, T, D, device="cuda")
+    outs = [qw, y]
+    head = (ptr(pre), dt, ptr(bias), ptr(denom), ptr(v), dt, ptr(g), ptr(w), ptr(qw), dt, ptr(x), ptr(y))
+    if prefill:
+        S, c = torch.empty(B, D, A, device="cuda"), torch.empty(B, A, device="cuda")
+        wb = lib.ulm_block_fm_prefill_workspace_bytes(B, T, A, D, dt)
+        ws = torch.empty(wb, device="cuda", dtype=torch.uint8)
+        call("ulm_block_fm_prefill", *head, ptr(S), ptr(c), ptr(ws), wb, B, T, A, D, nat.stream_of(pre))
+        outs += [S, c]
+    else:
+        sb, wb = lib.ulm_fm_saved_bytes(B, T, A, D, dt), lib.ulm_block_fm_fwd_workspace_bytes(B, T, A, D)
+        saved, ws = (torch.empty(n, device="cuda", dtype=torch.uint8) for n in (sb, wb))
+        call("ulm_block_fm_fwd", *head, ptr(saved), sb, ptr(ws), wb, B, T, A, D, nat.stream_of(pre))
+    return outs
+
+
+@pytest.mark.parametrize("prefill", [False, True])
+@pytest.mark.parametrize("path", ["pair", "chunked", "generic"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T", [1, 65, 200, 1030])
+def test_formed_address_alone_and_among_many(T, dtype, path, prefill, monkeypatch):
+    """One row (two chunks side by side) and among 140 of two slot blocks each (one): the same bits of w q, the
+    output and the decode state, and w q and c against float64. c: some ten fp32 roundings, and lam = exp(g) an ulp
+    off, 1.2e-7, over a mean lag of 1 / 0.03 positions; w q the same or its dtype's rounding (2^-8, 2^-11)."""
+    monkeypatch.setenv("ULM_FM_PATH", path)
+    B, A, D = 140, 96, 32
+    say(f"formed address of one row alone and among {B}, T={T} {dtype} {path} prefill={prefill}")
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    rn = lambda *s: torch.randn(*s, device="cuda", generator=gen)  # noqa: E731
+    pre, v, x, bias = rn(B, T, A).to(dtype), rn(B, T, D).to(dtype), rn(B, T, D), 0.2 * rn(A)
+    g, w, le, denom = torch.full((1,), -0.03, device="cuda"), torch.exp(rn(A)), torch.zeros(1, device="cuda"), rn(B, T)
+    call("ulm_addr_fwd", ptr(pre), nat.dtype_code(dtype), ptr(bias), ptr(le), None, ptr(denom), B * T, A, nat.stream_of(pre))
+    many = _block_rows(pre, bias, denom, v, g, w, x, prefill)
+    for b in (0, B - 1):
+        cut = lambda t: t[b:b + 1].contiguous()  # noqa: E731
+        alone = _block_rows(cut(pre), bias, cut(denom), cut(v), g, w, cut(x), prefill)
+        for i, (one, all_) in enumerate(zip(alone, many)):
+            assert torch.equal(one[0], all_[b]), (b, i)
+    z = (pre.double() + bias.double()).clamp(min=0).square()
+    r, lam = z / (1 + z.sum(-1, keepdim=True)), torch.exp(g.double())
+    want = _q64(r, lam, w.double()) * w.double()
+    tol = 1e-6 + 1.2e-7 / 0.03
+    rel = {torch.float32: tol, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    # fp16 keeps 2^-24 of absolute precision below 2^-14
+    assert ((many[0].double() - want).abs() <= rel * want.abs() * 1.01 + (2.0 ** -24 if dtype == torch.float16 else 0)).all()
+    if prefill:
+        n = torch.zeros_like(r[:, 0])
+        for t in range(T):
+            n = lam * n + (r[:, t - 1] if t else 0)
+        assert ((many[3].double() - (w.double() + n)).abs() <= tol * (w.double() + n)).all()

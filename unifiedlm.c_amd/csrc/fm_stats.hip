@@ -388,12 +388,10 @@ __global__ __launch_bounds__(256 * CW, 3) void fwd_stats_kernel(RS rs, const flo
         if (va && on && live > 0) {
             const size_t r0 = (bs * T + t0) * A;   // wave-uniform row offset
             if (q16n) {
-#pragma unroll
-                for (int i = 0; i < kSeg; ++i) {
-                    if (i >= live) break;
+                for (int i = 0; i < live; ++i) {   // this thread's own elements of the tiles
                     const size_t ro = r0 + static_cast<size_t>(i) * A;
-                    st_row(q16n + ro, 2u * ac, static_cast<uint16_t>(qpk[i / 2] >> (16 * (i % 2))));
-                    st_row(k16n + ro, 2u * ac, static_cast<uint16_t>(kpk[i / 2] >> (16 * (i % 2))));
+                    st_row(q16n + ro, 2u * ac, sq[j * kSeg + i][s]);
+                    st_row(k16n + ro, 2u * ac, sk[j * kSeg + i][s]);
                 }
             }
             if (j == 0) nck[(bs * NT + n) * A + a] = cj;
