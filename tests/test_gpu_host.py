@@ -264,3 +264,65 @@ def test_function_modes_see_the_registered_op():
     assert "ulm.block_fwd.default" in seen and torch.equal(got, ref)
     with torch.device("cuda"):
         assert kernel.block_eager(*args, 1e-5, torch.float32) is not None
+
+
+def _all_calls(dout, args, leaves, block):
+    """One pass through every eager entry: memory and block with their backwards, a prefill, then decode steps."""
+    q, fast = kernel.unified_memory(*leaves)
+    out = [q, fast, *torch.autograd.grad((q, fast), leaves, (0.1 * q.detach(), fast.detach()))]
+    y = kernel.unified_block(*args, 1e-5)
+    out += [y, *torch.autograd.grad(y, args, dout)]
+    y, s = block.prefill(args[0].detach())
+    out += [y]
+    for t in range(18):
+        out.append(block.step(y[:, t], s))
+    block.flush_state(s)
+    return [t.clone() for t in out + [s["S"], s["c"], s["r_prev"], s["buf"]]]
+
+
+def _problem(seed):
+    args, dout = _args(2, 150, 64, 128, 4, seed)
+    torch.manual_seed(seed)
+    return dout, args, _memory_leaves(False), UnifiedBlock(ModelArgs(dim=64, hidden_dim=128)).cuda()
+
+
+def test_on_another_stream():
+    """Every eager entry on a stream of the caller's, the inputs' writes and the outputs' reads on it too: the
+    same bits as on the default stream."""
+    say("the eager calls on another stream")
+    ref = _all_calls(*_problem(5))
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    for _ in range(3):
+        with torch.cuda.stream(stream):
+            torch.cuda._sleep(20_000_000)   # a launch on any other stream would run ahead of the inputs
+            got = _all_calls(*_problem(5))
+        stream.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, ref))
+
+
+def test_from_two_threads():
+    """Two threads, each with its stream, state and inputs, at once: each gets its own results."""
+    import threading
+    say("the eager calls from two threads at once")
+    refs = [_all_calls(*_problem(s)) for s in (5, 6)]
+    torch.cuda.synchronize()
+    problems = [_problem(s) for s in (5, 6)]
+    torch.cuda.synchronize()
+    got, start = [None, None], threading.Barrier(2)
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        start.wait()
+        with torch.cuda.stream(stream):
+            got[i] = [_all_calls(*problems[i]) for _ in range(5)]
+        stream.synchronize()
+    threads = [threading.Thread(target=work, args=(i,)) for i in (0, 1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i in (0, 1):
+        assert got[i] is not None
+        for one in got[i]:
+            assert all(torch.equal(a, b) for a, b in zip(one, refs[i]))
