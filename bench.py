@@ -15,7 +15,10 @@ are resident in HBM before the timed region. Prints one JSON line:
              each launch uses, against the 2516.6 TFLOP/s dense bf16 peak.
              The events run in a second pass of the same timed steps: an event
              record between two dependent kernels lengthens the gap between
-             them, so the pass that gives value carries none.
+             them, so the pass that gives value carries none. Timed launches
+             hold one product each: where the untimed steps take dscores and
+             dv in one launch (small shapes, pair_dual_kernel), the events
+             time the two launches that stand in for it.
              The algorithmic flops are those of the evaluation that runs: for
              the six block-pair products 6 (A + D) per causal pair (t, s) of a
              batch row (mfma_executed_tflops counts their whole 128 x 128 tiles,

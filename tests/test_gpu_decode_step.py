@@ -1,4 +1,4 @@
-"""The two-launch decode position for small states (ulm_decode_step) against
+"""The two-launch decode position (ulm_decode_step) against
 the per-kernel form of UnifiedBlock.step, position by position through two
 write-backs, and the calls it leaves to that form (needs an MI355X). Both are
 fp32 evaluations of the same sums in other orders: outputs, S, c and r_prev
@@ -79,7 +79,7 @@ def test_whole_model_takes_one_call(N, monkeypatch):
 
 
 def test_left_to_the_per_kernel_form():
-    """A large state, a strided state, a state and weights that disagree: nothing is touched."""
+    """Too many sequences, a strided state, a state and weights that disagree: nothing is touched."""
     block = _block(64, 128, 4, 1).layers[0]
     say("calls the two-launch step leaves alone")
     for N, change in ((257, None), (4, "strided"), (4, "short")):

@@ -2,16 +2,16 @@
 // GEMM calls, native launches and autograd nodes in C++, behind a Python module.
 //
 // A block's training step is about 30 launches of a few microseconds each at
-// small sizes; enqueued from Python through registered ops it took 735 us of
-// host time for 283 us of GPU work (8 x 200 positions of the default model's
-// widths in fp32), and takes about 390 us from here. The prefill of one prompt
-// of 117 positions at the 110M widths went 238 -> 143 us, a decode position of
-// the default model 244 -> 171 us. Everything here evaluates what kernel.py's
-// implementations evaluate, with the same native calls in the same order, and
-// without the interpreter's lock; a call that is not a plain eager one, or that
-// they would refuse, returns None and is left to them: tracing, functorch
-// transforms, forward-mode tangents, tensor subclasses, disagreeing shapes, other
-// dtypes and devices.
+// small sizes; enqueued from Python through registered ops it took 735 us of host
+// time for 283 us of GPU work (8 x 200 positions of the default model's widths in
+// fp32), and takes about 390 us from here. The prefill of one prompt of 117
+// positions at the 110M widths went 238 -> 143 us (now 154, with copies of the
+// session's matrices), a decode position of the default model 244 -> 171 us.
+// Everything here evaluates what kernel.py's implementations evaluate, with the
+// same native calls in the same order, and without the interpreter's lock; a call
+// that is not a plain eager one, or that they would refuse, returns None and is
+// left to them: tracing, functorch transforms, forward-mode tangents, tensor
+// subclasses, disagreeing shapes, other dtypes and devices.
 #include <ATen/ATen.h>
 #include <ATen/core/dispatch/Dispatcher.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>

@@ -1660,12 +1660,17 @@ int launch_pair_backward(const uint16_t *vR, const uint16_t *doR, const uint16_t
     static std::mutex side_mu;
     const std::lock_guard<std::mutex> lock(side_mu);
     SideStream *sd = nullptr;
-    // ... and where neither fills the device by itself, in the dscores launch
-    // instead: one launch less, no fork. One block fwd + bwd, us, as before / in
-    // one launch, at (dscores + dv) jobs of 128 x 128 tiles: B=32 T=256 D=288
-    // (288) 121 / 116; B=2 T=1024 D=768 (168) 162 / 151; B=4 T=999 D=768 (336,
-    // forked before) 180 / 173; B=8 T=1024 D=512 (544, forked) 200 / 194; but
-    // B=16 T=1024 D=288 (960, forked) 252 / 255, D=768 (1344, forked) 640 / 652.
+    // ... and in the dscores launch instead where that work does not outweigh
+    // them, or where neither product fills the device by itself: one launch
+    // less, no fork. us, two launches or forked / one launch, at (dscores + dv)
+    // jobs of 128 x 128 tiles.
+    // Below 2e9, whatever the jobs (the backward alone): B=12 T=1024 D=100 (528)
+    // 90.6 / 83.9; B=96 T=256 D=288 (864) 181.6 / 173.5; B=32 T=1024 D=40 (1408)
+    // 167.8 / 164.1; B=512 T=128 D=200 (1536) 233.4 / 229.0; B=1024 T=100 D=64
+    // (2048) 222.9 / 217.0.
+    // From 2e9 on, by the jobs (fwd + bwd): B=4 T=999 D=768 (336) 180 / 173;
+    // B=8 T=1024 D=512 (544) 200 / 194; but B=16 T=1024 D=288 (960) 252 / 255,
+    // D=768 (1344) 640 / 652.
     const double work = static_cast<double>(B) * Tq * Tq * D;
     const int jobs = B * MT * (MT + 1) / 2 + B * MT * ((D + 127) / 128);
     const bool dual = (work < 2e9 || jobs <= 640) && !la_timer_on();

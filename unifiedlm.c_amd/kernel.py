@@ -675,6 +675,8 @@ def matrix_copies(device, *mats):
     launch: 9 us of a 117-position prompt's 154 for a block's three (17 by way of
     torch.cat in Python, which serves tensors the host module leaves alone)."""
     device = torch.device(device)
+    if device.type == "cuda" and device.index is None:
+        device = torch.device("cuda", torch.cuda.current_device())
     if device.type == "cuda" and all(m.device == device for m in mats) and _plain_eager():
         out = nat.host().copies(*mats)
         if out is not None:
@@ -761,8 +763,8 @@ def decode_step(x, states, norm_eps):
     decode states (dicts of buf, S, c, r_prev, pv and pr, the pending count
     "np" and the parameters "params"), norm_eps their norms' epsilons. The
     states are updated in place. Returns the last block's output, or None,
-    with nothing touched, for a call this form does not take (large states,
-    other dtypes or layouts, tensors that disagree with each other): the
+    with nothing touched, for a call this form does not take (sizes at which
+    the per-kernel form is the faster one, other dtypes or layouts, tensors that disagree with each other): the
     per-kernel form serves those, or refuses them."""
     return nat.host().decode_step(x, states, norm_eps) if _plain_eager() else None
 

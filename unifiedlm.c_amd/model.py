@@ -172,7 +172,7 @@ class UnifiedBlock(nn.Module):
     @torch.no_grad()
     def init_state(self, batch: int, device):
         """The decode state before the first position (S = 0, c = w, no
-        previous address, an empty conv window) with the parameter copies."""
+        previous address, an empty conv window) with what _step_params takes."""
         width, slots = self.mu.out_features, self.mu.in_features
         params = self._step_params(device)
         zeros = lambda *shape: torch.zeros(*shape, device=device, dtype=torch.float32)
@@ -237,8 +237,10 @@ class UnifiedBlock(nn.Module):
         appends its term and reads S with the terms added, and the position
         that fills the last term writes S back with all of them. The maths of
         model.py:107-109 in another order: S moves one write per
-        DECODE_PENDING positions instead of one per position. A small
-        batch of it takes two launches in all (kernel.decode_step)."""
+        DECODE_PENDING positions instead of one per position. Few sequences
+        take two launches in all (kernel.decode_step), which updates every
+        tensor of the state in place, s["r_prev"] too: what a caller wants to
+        keep of a state it copies."""
         p = s["params"]
         x32 = x.float().contiguous()
         N, width, slots = s["S"].shape
