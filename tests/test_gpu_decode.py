@@ -71,3 +71,21 @@ def test_deferred_state_matches_direct(N, D, A):
             say(f"  write-back at position {t}: state rel {serr:.2e}, output rel {err:.2e}")
             assert serr < 1e-6, (t, serr)
             m = 0
+
+
+@pytest.mark.parametrize("N,D,A", [(24, 70, 1024), (33, 130, 3072), (130, 65, 520), (9, 100, 4096), (300, 64, 260)])
+def test_write_back_rows_alone_and_among_many(N, D, A):
+    """The write-back takes 8 or 64 rows per workgroup, by the batch: a sequence alone and among N, the same bits."""
+    say(f"write-back of one sequence alone and among {N}, D={D} A={A}")
+    gen = torch.Generator(device="cuda").manual_seed(N + A)
+    rn = lambda *s: torch.randn(*s, device="cuda", generator=gen)  # noqa: E731
+    S, pv, pr, q = rn(N, D, A), rn(16, N, D), rn(16, N, A).abs() / A, rn(N, A).abs()
+    g, x, y = torch.tensor([-0.05], device="cuda"), rn(N, D), rn(N, D)
+    for m in (1, 16):
+        many = S.clone()
+        out = kernel.decode_deferred(many, pv, pr, m, True, q, g, x, y)
+        for n in (0, N - 1):
+            cut = lambda t: t[n:n + 1].clone()  # noqa: E731
+            one = cut(S)
+            o = kernel.decode_deferred(one, pv[:, n:n + 1].contiguous(), pr[:, n:n + 1].contiguous(), m, True, cut(q), g, cut(x), cut(y))
+            assert torch.equal(one[0], many[n]) and torch.equal(o[0], out[n])

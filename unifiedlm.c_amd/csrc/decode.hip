@@ -346,12 +346,32 @@ __global__ __launch_bounds__(256) void decode_read_kernel(const float *__restric
     }
 }
 
-// Rows (features) per workgroup of a write-back: 64 where that leaves 1024
-// workgroups (each re-reads its sequence's pending keys, 12 KB a key at 3072
-// slots), else 8, since fewer workgroups leave CUs idle: at 8 sequences of the
-// 110M widths 64 rows make 96 workgroups and the launch took 76 us for 150 MB.
+// Rows (features) per workgroup of a write-back: 64, or 8 where 64 fill at most
+// half of the device, or leave under 1024 workgroups and the pending keys that an
+// XCD's workgroups read stay in its L2. A workgroup reads its sequence's keys
+// (16 A floats) for its rows, so 8 rows read as many bytes of keys as of state:
+// from L2 that costs nothing, from beyond it more than the shorter last round of
+// workgroups gives. Consecutive workgroups are consecutive sequences, so an XCD
+// meets an eighth of them where their number is a multiple of 8, else all.
+// Past 12 waves (3072 slots) 8 rows gain where they fill idle CUs alone.
+// us at 64 rows / 8, at (sequences, features, slots), with the share of the
+// device that 64 rows fill (rounds of workgroups) and the keys per XCD:
+//   (8, 768, 3072)     0.4    74 / 38           (16, 768, 3072)   0.8  0.4 MB   81 / 70
+//   (150, 128, 712)    0.3    70 / 31           (24, 768, 3072)   1.1  0.6     155 / 101
+//   (500, 64, 712)     0.5    73 / 60           (72, 768, 3072)   3.4  1.8     321 / 284
+//   (8, 768, 4096)     0.4    91 / 54           (120, 512, 3072)  3.8  2.9     329 / 329
+//   (25, 512, 3072)    0.8    85 / 94, 4.9 MB   (256, 192, 3072)  3.0  6.3     273 / 380
+//   (13, 1024, 4096)   0.8   107 / 123, 3.4     (85, 768, 3072)   4.0  17      354 / 536
 constexpr int kFlushRows = 64, kFlushRowsFew = 8;
-constexpr int kFlushWgs = 1024;
+constexpr size_t kFlushWgs = 1024, kFlushKeys = 3400000;   // bytes; an XCD's L2 is 4 MB
+constexpr size_t kCus = 256, kXcds = 8;
+
+bool flush_few(size_t N, int D, int A) {
+    const size_t wgs = N * ((D + kFlushRows - 1) / kFlushRows), waves = (A / 4 + kWave - 1) / kWave;
+    const size_t resident = kCus * ((waves <= 12 ? 12 : 16) / waves);   // workgroups at once, by their registers
+    const size_t keys = 4 * kMaxPending * A * (N % kXcds ? N : N / kXcds);
+    return 2 * wgs <= resident || (waves <= 12 && wgs < kFlushWgs && keys <= kFlushKeys);
+}
 // rows whose loads a lane has in flight at once: 8 where the registers allow
 // (12 waves, 168 VGPRs), else 4
 template <int MAXW> constexpr int flush_batch() { return MAXW <= 12 ? 8 : 4; }
@@ -442,7 +462,7 @@ template <bool OUT>
 int launch_flush(float *S, const float *pv, const float *pr, int m, const float *q, const float *g, const float *x,
                  const float *ymu, float *out, int N, int D, int A, hipStream_t s) {
     const int waves = (A / 4 + kWave - 1) / kWave;   // one 256-slot strip per wave
-    const bool few = static_cast<size_t>(N) * ((D + kFlushRows - 1) / kFlushRows) < kFlushWgs;
+    const bool few = flush_few(N, D, A);
     const int rows = few ? kFlushRowsFew : kFlushRows;
     const dim3 grid(N, (D + rows - 1) / rows), wg(waves * kWave);
     if (waves <= 12 && few)
