@@ -121,3 +121,32 @@ def test_formed_address_alone_and_among_many(T, dtype, path, prefill, monkeypatc
         for t in range(T):
             n = lam * n + (r[:, t - 1] if t else 0)
         assert ((many[3].double() - (w.double() + n)).abs() <= tol * (w.double() + n)).all()
+
+
+@pytest.mark.parametrize("w", [3e38, 9e37, 5e37, 1.5e36, 1e36, 1e-36, 8e-37, 7e-37, 2e-38, 1e-38, 1e-39])
+def test_quotients_of_huge_and_tiny_masses(w):
+    """A wave of one such mass: r / c as a division gives it, quotients below 2^-126 and reciprocals there included."""
+    say(f"forward statistics: every prior mass {w}")
+    T, A = 70, 64
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    r = torch.zeros(1, T, A, device="cuda")
+    r[0, T - 1] = torch.rand(A, device="cuda", generator=gen) * 2.0 ** torch.randint(-20, 1, (A,), device="cuda", generator=gen)
+    w = torch.full((A,), w, device="cuda")
+    q, _ = unified_memory(r, torch.ones(1, T, 4, device="cuda"), torch.tensor(-0.5, device="cuda"), w)
+    want = (r[0, T - 1].double() / w.double()).float()
+    got, fin = q[0, T - 1], torch.isfinite(want)
+    assert torch.equal(torch.isinf(got), ~fin)   # overflows as a division's
+    # an ulp of the quotient (2^-149 below 2^-126)
+    assert ((got[fin].double() - want[fin].double()).abs() <= want[fin].double() * 2.0 ** -23 + 2.0 ** -149).all()
+
+
+def test_keys_whose_sum_nears_the_largest_float():
+    """A key of 1e38 makes the masses after it huge and their quotients denormal; the reads through the same key are of
+    ordinary size and want those quotients."""
+    say("forward statistics: a huge key")
+    T, A = 40, 32
+    r = torch.rand(1, T, A, device="cuda") / A
+    r[0, 3] = 1e38
+    q, _ = unified_memory(r, torch.ones(1, T, 4, device="cuda"), torch.tensor(-0.01, device="cuda"), torch.ones(A, device="cuda"))
+    ref = _q64(r.double(), torch.exp(torch.tensor(-0.01, device="cuda").double()), torch.ones(A, device="cuda").double())
+    assert ((q.double() - ref).abs() <= 2e-6 * ref + 2.0 ** -149).all()

@@ -150,8 +150,8 @@ template <class E> __device__ __forceinline__ void buf_store(E v, rsrc_t r, uint
     else __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, v), r, off, 0, 0);
 }
 
-// num / den to within an ulp, from den's reciprocal and one correction, for
-// normal den; zeros, infinities and NaN as a division has them
+// num / den to within an ulp, from den's reciprocal and one correction, where den
+// and its reciprocal are normal; zeros, infinities and NaN as a division has them
 __device__ __forceinline__ float quotient(float num, float den) {
     const float rc = __builtin_amdgcn_rcpf(den), q0 = num * rc;
     return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-den, q0, num), rc, q0), den, num);
@@ -327,13 +327,14 @@ __global__ __launch_bounds__(256 * CW, 3) void fwd_stats_kernel(RS rs, const flo
         // n before this thread's segment: the group's earlier segments, in order
         float cj = carry;
         for (int m = 0; m < js; ++m) cj = lam16 * cj + tot[m][s];
-        float pw = lam, qt[kSeg], least = 3.0e38f;
+        float pw = lam, qt[kSeg], least = 3.0e38f, most = 0.f;
         uint32_t qpk[kSeg / 2], kpk[kSeg / 2];   // bf16 pairs of this thread's 16 positions
 #pragma unroll
         for (int i = 0; i < kSeg; ++i) {
             nl[i] = wa + (pw * cj + nl[i]);   // c
             pw *= lam;
             least = fminf(least, fabsf(nl[i]));
+            most = fmaxf(most, fabsf(nl[i]));
         }
         if (c_last && on && va && live > 0 && t0 + live == T) {
             float cl = nl[0];
@@ -341,7 +342,7 @@ __global__ __launch_bounds__(256 * CW, 3) void fwd_stats_kernel(RS rs, const flo
             for (int i = 1; i < kSeg; ++i) cl = i < live ? nl[i] : cl;
             c_last[bs * A + a] = cl;
         }
-        if (__any(least < 0x1p-120f)) {   // a prior mass next to nothing: its reciprocal may overflow
+        if (__any(least < 0x1p-120f || most > 0x1p120f)) {   // a mass whose reciprocal may overflow, or lose bits below 2^-126
 #pragma unroll
             for (int i = 0; i < kSeg; ++i) qt[i] = rv[i] / nl[i];
         } else {
