@@ -356,11 +356,12 @@ int ulm_decode_read(const float *S, const float *pv, const float *cj, int m, con
 int ulm_decode_flush(float *S, const float *pv, const float *pr, int m, const float *q, const float *g,
                      const float *x, const float *ymu, float *out, int N, int D, int A, void *stream);
 
-/* One position of n_layers consecutive blocks for up to 256 sequences whose
- * states are small (up to 320 MB per block, and less for many sequences:
- * ulm_decode_step_workspace_bytes() tells), two launches per block (a third
- * where a block's 16th term makes it write its state back): what the per-kernel entries above and the three projections
- * compute, on the same deferred state. x (N,D) is the first block's input,
+/* One position of n_layers consecutive blocks for up to 256 sequences, at the
+ * sizes where two launches per block take less time than the entries above
+ * (ulm_decode_step_workspace_bytes() tells: states of at most 320 MB per block,
+ * less for many sequences). A third launch where a block's 16th term makes it
+ * write its state back. What the per-kernel entries above and the three
+ * projections compute, on the same deferred state. x (N,D) is the first block's input,
  * out (N,D) the last one's output, neither aliasing the other.
  * A layer names a block's parameters, fp32 and contiguous: norm_w (D,),
  * conv_w (D,Kc), key_w (A,D), key_b (A,), log_eps (1,), val_w (D,D),

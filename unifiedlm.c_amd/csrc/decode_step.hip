@@ -35,7 +35,6 @@ namespace step {
 
 constexpr int kMaxPending = 16;   // as decode.hip
 constexpr int kMaxN = 256;        // sequences
-constexpr size_t kMaxState = 320u << 20;   // bytes of S_base
 // Microseconds up to which a block's position takes this form (cost below): the
 // per-kernel form's eight calls take 88 of host time, whatever their sizes, and
 // from about 250 MB of state on 94 of the device's. 16 positions of one block, us,
@@ -499,7 +498,7 @@ using namespace ulm;
 // the shapes this form takes; at least one sequence's u fits the LDS of a workgroup
 static bool step_supported(int N, int D, int A, int Kc) {
     return N >= 1 && N <= step::kMaxN && D >= 1 && A >= 4 && A % 4 == 0 && A <= 4096 && Kc >= 1 && Kc <= step::kMaxTaps &&
-           step::in_groups(N, D) > 0 && 4ull * N * D * A <= step::kMaxState && step::cost(N, D, A) <= step::kMaxCost;
+           step::in_groups(N, D) > 0 && step::cost(N, D, A) <= step::kMaxCost;
 }
 
 extern "C" size_t ulm_decode_step_workspace_bytes(int N, int D, int A, int Kc) {
